@@ -40,6 +40,8 @@ extern "C" int gd_gdn_gate(gd_ctx *ctx, const float *bPre, const float *aPre, co
 
 // One thread per channel; the ring stays in registers across the N tokens.
 // window = [ring[0..dConv-2], x]; out = silu(sum window[j] * cw[c*dConv + j]).
+// Serial over the tokens: every x of a channel is read before the outputs
+// after it are written, so out may overlap x (the tiled kernel below may not).
 template <int KC>
 __global__ void gd_conv_kernel(const float *x, float *ring, const float *cw, float *out,
                                int convDim, int64_t N) {
@@ -65,6 +67,125 @@ __global__ void gd_conv_kernel(const float *x, float *ring, const float *cw, flo
     for (int j = 0; j + 1 < KC; j++) ring[(int64_t)j * convDim + c] = r[j];
 }
 
+// V consecutive floats.
+template <int V> struct Floats { float v[V]; };
+template <int V> __device__ __forceinline__ Floats<V> ld_floats(const float *p) {
+    Floats<V> r;
+    if constexpr (V == 4) {
+        const f32x4 a = *(const f32x4 *)p;
+#pragma unroll
+        for (int i = 0; i < 4; i++) r.v[i] = a[i];
+    } else {
+        r.v[0] = *p;
+    }
+    return r;
+}
+template <int V> __device__ __forceinline__ void st_floats(float *p, const Floats<V> &r) {
+    if constexpr (V == 4) *(f32x4 *)p = f32x4{r.v[0], r.v[1], r.v[2], r.v[3]};
+    else *p = r.v[0];
+}
+
+// The same conv with the tokens in tiles of TT: a thread holds V channels and
+// slides its window over the tile, its TT + KC - 1 input rows all requested
+// before the first is used.  Memory-bound (x read and out written once, plus
+// the KC - 1 rows a tile reads of the one before it): 1000 tokens x 10240
+// channels 327 us with one thread per channel walking all tokens (40
+// workgroups, one load in flight each), 20 us here (4.1 TB/s of x and out; a
+// large copy runs at 4.7).  Only tile 0 reads the ring
+// (TT >= KC - 1), so it alone advances it, after its reads.
+template <int KC, int V, int TT>
+__global__ __launch_bounds__(256) void gd_conv_tile_kernel(const float *__restrict__ x, float *ring,
+                                                           const float *__restrict__ cw,
+                                                           float *__restrict__ out, int convDim,
+                                                           int64_t N) {
+    static_assert(TT >= KC - 1, "only tile 0 may reach back into the ring");
+    const int c = (blockIdx.x * 256 + threadIdx.x) * V;
+    if (c >= convDim) return;
+    const int64_t n0 = (int64_t)blockIdx.y * TT;
+    Floats<V> win[TT + KC - 1], old[KC];                 // win[j]: token n0 - (KC - 1) + j
+    float w[V][KC];
+#pragma unroll
+    for (int j = 0; j < TT + KC - 1; j++) {
+        const int64_t m = n0 - (KC - 1) + j;
+        win[j] = ld_floats<V>(x + (m < 0 ? 0 : m < N ? m : N - 1) * convDim + c);
+    }
+#pragma unroll
+    for (int i = 0; i < V; i++)
+#pragma unroll
+        for (int j = 0; j < KC; j++) w[i][j] = cw[(int64_t)(c + i) * KC + j];
+    if (n0 == 0) {
+#pragma unroll
+        for (int j = 0; j + 1 < KC; j++) {
+            old[j] = ld_floats<V>(ring + (int64_t)j * convDim + c);
+            win[j] = old[j];
+        }
+    }
+#pragma unroll
+    for (int t = 0; t < TT; t++) {
+        if (n0 + t >= N) break;
+        Floats<V> y;
+#pragma unroll
+        for (int i = 0; i < V; i++) {
+            float acc = 0.0f;
+#pragma unroll
+            for (int j = 0; j < KC; j++) acc += win[t + j].v[i] * w[i][j];
+            y.v[i] = gd_silu(acc);
+        }
+        st_floats<V>(out + (n0 + t) * convDim + c, y);
+    }
+    if (n0 == 0) {
+        // The inputs of tokens N - KC + 1 .. N - 1 (the old ring's where those
+        // precede token 0: row KC - 1 + m).
+#pragma unroll
+        for (int j = 0; j + 1 < KC; j++) {
+            const int64_t m = N - (KC - 1) + j;
+            Floats<V> r;
+            if (m >= 0) {
+                r = ld_floats<V>(x + m * convDim + c);
+            } else {
+                r = old[0];
+#pragma unroll
+                for (int k = 1; k + 1 < KC; k++)
+                    if (KC - 1 + m == k) r = old[k];
+            }
+            st_floats<V>(ring + (int64_t)j * convDim + c, r);
+        }
+    }
+}
+
+// The tiled conv where nothing the tiles write is read by another tile: out
+// and ring apart from each other and from the inputs.  Four channels a thread
+// where rows keep 16-byte alignment.  Tiles of 16 tokens (a fifth more rows
+// read than the input has) once they fill the chip twice over, else of 4 (8
+// where the window is longer), so that short inputs spread over more CUs.
+template <int KC>
+static bool launch_conv_tiles(gd_ctx *ctx, const float *x, float *ring, const float *cw, float *out,
+                              int convDim, int64_t N) {
+    auto apart = [](const void *a, size_t an, const void *b, size_t bn) {
+        const uintptr_t p = (uintptr_t)a, q = (uintptr_t)b;
+        return p + an <= q || q + bn <= p;
+    };
+    const size_t xb = (size_t)N * convDim * 4, rb = (size_t)(KC - 1) * convDim * 4, wb = (size_t)convDim * KC * 4;
+    if (!apart(x, xb, out, xb) || !apart(cw, wb, out, xb)) return false;
+    if (KC > 1 && !(apart(ring, rb, out, xb) && apart(ring, rb, x, xb) && apart(ring, rb, cw, wb)))
+        return false;
+    constexpr int TS = KC <= 5 ? 4 : 8, TL = 16;
+    const bool vec = convDim % 4 == 0 &&
+                     (((uintptr_t)x | (uintptr_t)out | (KC > 1 ? (uintptr_t)ring : 0)) & 15) == 0;
+    const unsigned gx = gd_blocks(convDim, vec ? 1024 : 256);
+    const int cus = ctx->num_cus > 0 ? ctx->num_cus : 256;
+    const bool large = (int64_t)gx * ((N + TL - 1) / TL) >= 2 * cus;
+    const int64_t gy = (N + (large ? TL : TS) - 1) / (large ? TL : TS);
+    if (gy > 65535) return false;
+    const dim3 g(gx, (unsigned)gy), b(256);
+#define GD_CONV_TILE(V_, T_) hipLaunchKernelGGL((gd_conv_tile_kernel<KC, V_, T_>), g, b, 0, ctx->stream, \
+                                                x, ring, cw, out, convDim, N)
+    if (vec) { if (large) GD_CONV_TILE(4, TL); else GD_CONV_TILE(4, TS); }
+    else { if (large) GD_CONV_TILE(1, TL); else GD_CONV_TILE(1, TS); }
+#undef GD_CONV_TILE
+    return true;
+}
+
 extern "C" int gd_gdn_conv(gd_ctx *ctx, const float *qkvMix, float *convState, const float *cw,
                            float *out, int convDim, int dConv, int64_t N) {
     GD_CHECK_CTX(ctx);
@@ -75,8 +196,9 @@ extern "C" int gd_gdn_conv(gd_ctx *ctx, const float *qkvMix, float *convState, c
     dim3 g(gd_blocks(convDim, 256)), b(256);
     switch (dConv) {
 #define GD_CONV_CASE(KC) \
-    case KC: hipLaunchKernelGGL(gd_conv_kernel<KC>, g, b, 0, ctx->stream, qkvMix, convState, cw, \
-                                out, convDim, N); break;
+    case KC: if (!launch_conv_tiles<KC>(ctx, qkvMix, convState, cw, out, convDim, N)) \
+            hipLaunchKernelGGL(gd_conv_kernel<KC>, g, b, 0, ctx->stream, qkvMix, convState, cw, \
+                               out, convDim, N); break;
         GD_CONV_CASE(1) GD_CONV_CASE(2) GD_CONV_CASE(3) GD_CONV_CASE(4)
         GD_CONV_CASE(5) GD_CONV_CASE(6) GD_CONV_CASE(7) GD_CONV_CASE(8)
 #undef GD_CONV_CASE

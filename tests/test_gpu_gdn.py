@@ -53,6 +53,29 @@ def test_conv(ctx, N):
     assert rel_diff(ctx.get(dr, ring.size, np.float32), ring_ref) < 1e-6
 
 
+@pytest.mark.parametrize("convDim,kc,N,off", [
+    (260, 4, 2, 0), (260, 4, 3, 0), (260, 4, 5, 0), (1028, 4, 17, 0), (257, 4, 33, 0),
+    (256, 4, 21, 1), (512, 1, 9, 0), (512, 2, 1, 0), (512, 8, 3, 0), (516, 8, 7, 0), (512, 8, 19, 0),
+    (1024, 4, 8200, 0), (1024, 8, 8193, 0)])
+def test_conv_tiles(ctx, convDim, kc, N, off):
+    """Token tiles of every length (shorter than the window, one short of and
+    past whole tiles, long ones), rows off 16-byte alignment (off), and a call
+    whose output replaces its input: each output and the ring against the
+    token-serial oracle."""
+    x = O.lcg_normal(N * convDim, 31).reshape(N, convDim)
+    ring = O.lcg_normal(max(kc - 1, 1) * convDim, 32)
+    cw = O.lcg_uniform(convDim * kc, 33, -0.5, 0.5)
+    ring_ref = ring[:(kc - 1) * convDim].copy()
+    want = O.gdn_conv(x, ring_ref, cw, convDim, kc)
+    dx, dw, do = ctx.alloc(x.nbytes + 16) + 4 * off, ctx.put(cw), ctx.alloc(x.nbytes + 16) + 4 * off
+    for out in (do, dx):
+        dr = ctx.put(ring)
+        ctx.set(dx, x)
+        ctx.gd_gdn_conv(dx, dr, dw, out, convDim, kc, N)
+        assert rel_diff(ctx.get(out, (N, convDim), np.float32), want) < 1e-5
+        assert np.array_equal(ctx.get(dr, ring_ref.size, np.float32), ring_ref)
+
+
 def test_norms_and_elementwise(ctx):
     N, nK, d, convDim = 9, 16, 128, 6144
     x = O.lcg_normal(N * convDim, 21).reshape(N, convDim)
