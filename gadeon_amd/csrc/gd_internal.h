@@ -217,6 +217,28 @@ __device__ __forceinline__ uint16_t gd_f2h(float x) {
     return __builtin_bit_cast(uint16_t, (f16)x);   // RNE
 }
 
+// x = hi + lo with hi = f16(x), lo = f16(x - hi): about 22 bits.  x is made
+// opaque first: where it is a product, the compiler otherwise rounds the exact
+// product to f16 in one place (v_fma_mixlo) and its f32 rounding in another,
+// and where the two differ by an f16 ulp hi and lo no longer belong together
+// (one element in some ten thousand off by 2^-12).
+__device__ __forceinline__ void gd_split_f16(float x, f16 &hi, f16 &lo) {
+    asm("" : "+v"(x));
+    hi = (f16)x;
+    lo = (f16)(x - (float)hi);
+}
+// Two values in four instructions: packed conversions and mixed-precision
+// fmas (the -1 is opaque: as a constant it folds the fma back into a
+// conversion and a subtraction).
+__device__ __forceinline__ void gd_split2_f16(float x, float y, f16x2 &hi, f16x2 &lo) {
+    asm("" : "+v"(x), "+v"(y));
+    typedef float f32x2 __attribute__((ext_vector_type(2)));
+    float m1 = -1.0f;
+    asm("" : "+s"(m1));
+    hi = __builtin_convertvector((f32x2{x, y}), f16x2);
+    lo = __builtin_convertvector((f32x2{fmaf((float)hi[0], m1, x), fmaf((float)hi[1], m1, y)}), f16x2);
+}
+
 __device__ __forceinline__ float gd_silu(float x) { return x / (1.0f + expf(-x)); }
 __device__ __forceinline__ float gd_sigmoid(float x) { return 1.0f / (1.0f + expf(-x)); }
 // Stable softplus, relu(x) + log1p(exp(-|x|)) (Kernels.swift:7-10).

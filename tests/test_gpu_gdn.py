@@ -216,6 +216,33 @@ def test_prefill_chunked_vs_sequential(ctx, T, nV, nK, C, io, s0):
     assert rel_diff(ctx.get(dS_, S.size, np.float32), S_ref) < 2e-3
 
 
+@pytest.mark.parametrize("T,nV,nK,C,io,pad,off", [
+    (31, 6, 2, 64, ga.F16, 0, 0), (33, 2, 4, 32, ga.F32, 3, 4), (64, 2, 1, 16, ga.F32, 0, 0),
+    (97, 6, 2, 64, ga.F16, 5, 2), (200, 3, 3, 64, ga.F32, 0, 0)])
+def test_prefill_weak_decay(ctx, T, nV, nK, C, io, pad, off):
+    """Gates near 1 carry the state through every chunk (at the usual draws a
+    chunk forgets it), over whole and ragged chunks, value heads sharing key
+    heads and key heads without a value head, and outputs whose rows are off
+    16-byte alignment (pad, off): o (in the caller's type) and S against the
+    f64 scan.  f32 outputs and S within 2e-5: operands of 22 bits, T x 1.5e-7
+    in the sums of up to 200 tokens; f16 outputs within their rounding."""
+    dS, esz = 128, 2 if io == ga.F16 else 4
+    q, k, v, g, beta, S = prefill_inputs(T, nV, nK, dS, 150 + T, 0.5)
+    g = (g * np.float32(0.01)).astype(np.float32)
+    cv = (lambda a: a.view(np.uint16)) if io == ga.F16 else (lambda a: a.astype(np.float32))
+    stride = nV * dS + pad
+    dS_, do = ctx.put(S), ctx.alloc(T * stride * esz + 16) + off
+    ctx.gd_gdn_prefill(T, nV, nK, dS, dS, ctx.put(cv(q)), nK * dS, ctx.put(cv(k)), nK * dS, ctx.put(cv(v)),
+                       nV * dS, io, ctx.put(g), ctx.put(beta), dS_, do, stride, io, 1 / np.sqrt(dS), C)
+    S_ref = S.astype(np.float32).copy()
+    o_ref = O.gdn_sequential(q.astype(np.float32), k.astype(np.float32), v.astype(np.float32),
+                             g, beta, S_ref, np.float32(1 / np.sqrt(dS)))
+    rows = ctx.get(do, T * stride - pad, np.float16 if io == ga.F16 else np.float32)
+    o = np.stack([rows[t * stride:t * stride + nV * dS] for t in range(T)]).reshape(T, nV, dS)
+    assert rel_diff(o, o_ref) < (6e-4 if io == ga.F16 else 2e-5)
+    assert rel_diff(ctx.get(dS_, S.size, np.float32), S_ref) < 2e-5
+
+
 @pytest.mark.parametrize("dS", [128, 64, 96, 256, 48])
 def test_scan_batch_conv_layout(ctx, dS):
     """MetalEnc.gdnScanBatch's packed convOut[N][q|k|v] layout (MetalEnc.swift:741-778),
