@@ -13,11 +13,13 @@
 // which is how a HIP caller would lay pages out.
 //
 // MI355X design:
-//   * Decode (one query): flash decoding, DSPLIT key splits per head; each
-//     wave takes whole keys, a lane holding HD/64 consecutive dims, with an
-//     online softmax; a block merges its waves and writes (max, sum,
-//     acc[HD]); a combine kernel merges the splits with the output gate.  The
-//     stack's variant folds in the per-token preparation (split of q|gate,
+//   * Decode (one query), gd_attn_paged: flash decoding on the matrix cores,
+//     a kv head's keys read once for all its q heads (k_attn_paged).
+//   * Decode, the stack's variant (k_attn_decode): flash decoding, DSPLIT key
+//     splits per head; each wave takes whole keys, a lane holding HD/64
+//     consecutive dims, with an online softmax; a block merges its waves and
+//     writes (max, sum, acc[HD]); a combine kernel merges the splits with the
+//     output gate.  It folds in the per-token preparation (split of q|gate,
 //     RMS norm, partial NEOX rope, the cache append), so the new key never
 //     round-trips through the cache within the step.
 //   * Prefill (N queries): flash attention on the matrix cores, block (head,
@@ -30,6 +32,7 @@
 //     the projection rows itself and prep handles the kv heads only.
 #include "gd_internal.h"
 
+#include <algorithm>
 #include <type_traits>
 
 namespace {
@@ -414,27 +417,24 @@ __global__ __launch_bounds__(256) void k_attn_prefill(
 
 // ---------------------------------------------------------------- decode
 
-// Decode attention for one query token, split over keys (flash decoding):
-// block (head h, split sp) of 2 HD threads (NWD = HD / 32 waves).
-//   FUSED (the stack): the block prepares its own q from the projection row
-//   (q of head h at h qs: the q half of a [q | gate] pair when qs = 2 HD,
-//   plain q when qs = HD; RMS norm, rope; threads 0..HD-1) and the
-//   new k and v (threads HD..2HD-1), rounded to f16 as the cache stores them;
-//   the split that holds key pos uses them for that key instead of reading
-//   the cache, and the first q head of each kv group appends them.  No block
-//   reads the cache at pos.
-//   Otherwise (gd_attn_paged): q arrives prepared, the T keys lo .. T-1 are
-//   all cached.
-// Each wave takes whole keys j = lo + NWD sp + w + STEP i with a lane holding
+// The stack's decode attention for one query token, split over keys (flash
+// decoding): block (head h, split sp) of 2 HD threads (NWD = HD / 32 waves).
+// The block prepares its own q from the projection row (q of head h at h qs:
+// the q half of a [q | gate] pair when qs = 2 HD, plain q when qs = HD; RMS
+// norm, rope; threads 0..HD-1) and the new k and v (threads HD..2HD-1),
+// rounded to f16 as the cache stores them; the split that holds key pos uses
+// them for that key instead of reading the cache, and the first q head of
+// each kv group appends them.  No block reads the cache at pos.
+// Each wave takes whole keys j = NWD sp + w + STEP i with a lane holding
 // HD/64 consecutive dims, keeping an online-softmax partial; the block
 // merges its waves and writes (max, sum, acc[HD]) for the split; the combine
 // kernel merges the splits (Attention.swift:108-134).  A wave keeps the K
 // and V of its next KB keys in flight (a register ring), their page-table
 // entries one round ahead of them, so a key waits for neither.
-template <int HD, bool FUSED>
+template <int HD>
 __global__ __launch_bounds__(2 * HD) void k_attn_decode(
         const float *src, int qs, const float *q_norm, const float *k_norm, uint16_t *kc,
-        uint16_t *vc, const int32_t *page_table, const int32_t *pos_ptr, int T, int lo, float *part,
+        uint16_t *vc, const int32_t *page_table, const int32_t *pos_ptr, float *part,
         int H, int HKV, int block, float scale, int n_rot, float base, float eps,
         const float2 *rtab, int rtab_n) {
     constexpr int NT = 2 * HD, NWD = NT / 64, DPL = HD / 64, WPH = HD / 64;
@@ -445,10 +445,9 @@ __global__ __launch_bounds__(2 * HD) void k_attn_decode(
     const int h = blockIdx.x, sp = blockIdx.y, t = threadIdx.x;
     const int lane = t & 63, w = __builtin_amdgcn_readfirstlane(t >> 6);
     const int kvh = h / (H / HKV), kvDim = HKV * HD;
-    // Keys read from the cache: [lo, pos) for the stack (pos = the new
-    // token's position, taken from its registers), [lo, T) otherwise.
-    const int pos = FUSED ? *pos_ptr : T;
-    const bool has_pos = FUSED && sp == (pos / NWD) % DSPLIT;   // wave pos % NWD takes key pos
+    // Keys read from the cache: [0, pos), pos the new token's position.
+    const int pos = *pos_ptr;
+    const bool has_pos = sp == (pos / NWD) % DSPLIT;   // wave pos % NWD takes key pos
     // A lane's DPL f16 dims of one key: one dword (HD 128) or two (HD 256).
     using U = typename std::conditional<DPL == 2, uint32_t, u32x2>::type;
     auto ld = [&](const uint16_t *p) { return *(const U *)p; };
@@ -458,14 +457,13 @@ __global__ __launch_bounds__(2 * HD) void k_attn_decode(
     };
     // Cached keys of this wave: j0 + STEP i, i < nk.  Every load below is
     // unconditional (the compiler waits exactly only for straight-line
-    // loads): a key past the last reads position jlast instead, whose page
-    // exists (the new token's, or the last cached key's), and is not used.
-    const int j0 = lo + sp * NWD + w;
+    // loads): a key past the last reads position pos instead, whose page
+    // exists (the new token's), and is not used.
+    const int j0 = sp * NWD + w;
     const int nk = j0 < pos ? (pos - 1 - j0) / STEP + 1 : 0;
-    const int jlast = FUSED ? pos : T - 1;
     auto kpos = [&](int i) {
         const int jj = j0 + i * STEP;
-        return jj < pos ? jj : jlast;
+        return jj < pos ? jj : pos;
     };
     // Cache slots of keys i0 .. i0 + KB - 1, lane l holding key i0 + l % KB:
     // its page-table entry (a load) and its position in the page.
@@ -499,7 +497,7 @@ __global__ __launch_bounds__(2 * HD) void k_attn_decode(
         pg = entries(KB);
         __builtin_amdgcn_sched_barrier(0);
     };
-    if constexpr (FUSED) {
+    {
         // q of head h (hf = 0) and k of kv head kvh (hf = 1): RMS norm over
         // the head, then the partial NEOX rope, as k_attn_prep.
         const int H2 = H * qs;
@@ -539,11 +537,6 @@ __global__ __launch_bounds__(2 * HD) void k_attn_decode(
             kc[slot * kvDim + kvh * HD + i] = gd_f2h(y);
             vc[slot * kvDim + kvh * HD + i] = gd_f2h(vnew[i]);
         }
-    } else {
-        const float qx = t < HD ? src[(int64_t)h * HD + t] : 0.f;
-        prime();
-        if (t < HD) rot[0][t] = qx;
-        __syncthreads();
     }
     float qv[DPL], a[DPL];
 #pragma unroll
@@ -581,7 +574,7 @@ __global__ __launch_bounds__(2 * HD) void k_attn_decode(
 #pragma unroll
     for (int s = 0; s < KB; s++)
         if (i + s < nk) consume(kr[s], vr[s]);
-    if constexpr (FUSED) {
+    {
         // Key pos, from this block's own copy (f16, as cached).
         if (has_pos && w == pos % NWD) {
             uint32_t kw[DPL / 2], vw[DPL / 2];
@@ -619,6 +612,184 @@ __global__ __launch_bounds__(2 * HD) void k_attn_decode(
     }
 }
 
+// Decode attention over cached keys lo .. T-1 (gd_attn_paged) on the matrix
+// cores: workgroup (kv head, split sp of ns), the split's keys read once for
+// all of the kv head's q heads (8 of them a workgroup).  Wave w takes blocks
+// of 32 keys sp + ns (w + PW i): S^T = K Q^T with K straight from the cache as
+// the A operand, and O^T += V^T P^T with V staged as stored in the wave's own
+// LDS rows and read by the transposing LDS read (as k_attn_prefill; no
+// barrier in the loop).  The 16 columns of an MFMA are the eight heads' q as
+// f16 hi (columns 0..7) and lo (8..15), and P likewise, so both halves of a
+// product come from one instruction and are added across lanes lr, lr ^ 8.
+// Scores are in units of log2 (q is scaled by scale log2 e).  A block's K and
+// V are requested one block ahead, its page-table entries two.
+//   Bound by the latency of a few rounds of loads: one wave a key and q head,
+// with a wave reduction per key, took 42 us at 9001 keys of 24 / 4 heads x 256
+// (37 MB, each read by six heads' workgroups); this, on the 16 splits of
+// eight waves that the caller's scratch allows, 21 us (64 CUs), on 64 splits of
+// four 13; 32000 keys 27 us (4.9 TB/s of cache).
+constexpr int PW = 4;           // waves
+constexpr float LOG2E = 1.4426950408889634f;
+template <int HD>
+__global__ __launch_bounds__(64 * PW) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_attn_paged(
+        const float *q, const uint16_t *kc, const uint16_t *vc, const int32_t *page_table, int T,
+        int lo, float *part, int ns, int H, int HKV, int block, float scale) {
+    constexpr int KS = HD / 32, DT = HD / 16, VP = HD + 16;
+    constexpr int CPK = HD / 8;                           // 16-byte chunks of a key
+    constexpr int VCH = 32 * CPK / 64;                    // of a block's V, per lane
+    __shared__ __attribute__((aligned(16))) f16 Vs[PW][32][VP];
+    __shared__ f16x8 Qs[KS][64];
+    __shared__ float wm[PW][8], wl[PW][8];
+    static_assert(sizeof(Vs) >= (size_t)PW * 8 * HD * 4, "the merge reuses Vs");
+    const int G = H / HKV, groups = (G + 7) / 8;
+    const int kvh = blockIdx.x / groups, h0 = kvh * G + 8 * (blockIdx.x % groups);
+    const int nh = min(8, G - 8 * (int)(blockIdx.x % groups)), sp = blockIdx.y;
+    const int t = threadIdx.x, lane = t & 63, w = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int lr = lane & 15, g = lane >> 4, c = lr & 7;
+    const int64_t kvDim = (int64_t)HKV * HD;
+    const uint16_t *kb = kc + kvh * HD, *vb = vc + kvh * HD;
+    const int nb = (T - lo + 31) / 32;                    // key blocks
+    // Cache slot of key lane % 32 of block j (past the last key: the last).
+    auto slot_of = [&](int j) {
+        const int kp = min(lo + 32 * j + (lane & 31), T - 1);
+        return page_table[kp / block] * block + kp % block;
+    };
+    u32x4 kreg[2][KS], vreg[VCH];
+    auto fetchK = [&](int sl) {
+#pragma unroll
+        for (int kt = 0; kt < 2; kt++) {
+            const uint16_t *row = kb + __shfl(sl, 16 * kt + lr, 64) * kvDim + 8 * g;
+#pragma unroll
+            for (int ks = 0; ks < KS; ks++) kreg[kt][ks] = *(const u32x4 *)(row + 32 * ks);
+        }
+    };
+    auto fetchV = [&](int sl) {
+#pragma unroll
+        for (int n = 0; n < VCH; n++)
+            vreg[n] = *(const u32x4 *)(vb + __shfl(sl, (n * 64 + lane) / CPK, 64) * kvDim + 8 * (lane % CPK));
+    };
+    const int step = ns * PW;
+    int j = sp + ns * w;
+    int sl = slot_of(j), sn = slot_of(j + step);
+    // Q's operand, once per workgroup (it does not fit the registers beside
+    // a block of K and V and the sums at head dim 256).
+    for (int ks = w; ks < KS; ks += PW) {
+        const float *qrow = q + (int64_t)(h0 + min(c, nh - 1)) * HD + 32 * ks + 8 * g;
+        const f32x4 a = *(const f32x4 *)qrow, b = *(const f32x4 *)(qrow + 4);
+        const float qs = c < nh ? scale * LOG2E : 0.f;
+        f16x8 qf;
+#pragma unroll
+        for (int e = 0; e < 8; e++) {
+            f16 hi, lo_;
+            gd_split_f16((e < 4 ? a[e] : b[e - 4]) * qs, hi, lo_);
+            qf[e] = lr < 8 ? hi : lo_;
+        }
+        Qs[ks][lane] = qf;
+    }
+    fetchK(sl);
+    fetchV(sl);
+    f32x4 acc[DT];                                        // O^T rows 16 dt + 4 g + v
+#pragma unroll
+    for (int dt = 0; dt < DT; dt++) acc[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
+    float m = -INFINITY, l = 0.f;                         // l: this lane's keys only
+    __syncthreads();
+    for (; j < nb; j += step) {
+        f32x4 sc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+        for (int ks = 0; ks < KS; ks++) {
+            const f16x8 qf = Qs[ks][lane];
+#pragma unroll
+            for (int kt = 0; kt < 2; kt++)
+                sc[kt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, kreg[kt][ks]), qf, sc[kt],
+                                                                0, 0, 0);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        const int s2 = slot_of(j + 2 * step);
+        fetchK(sn);
+#pragma unroll
+        for (int n = 0; n < VCH; n++)
+            *(u32x4 *)&Vs[w][(n * 64 + lane) / CPK][8 * (lane % CPK)] = vreg[n];
+        fetchV(sn);
+        sn = s2;
+        __builtin_amdgcn_sched_barrier(0);
+        // hi + lo of a head's score; keys 16 kt + 4 g + v of the block.
+        float bmax = -INFINITY;
+#pragma unroll
+        for (int kt = 0; kt < 2; kt++)
+#pragma unroll
+            for (int v = 0; v < 4; v++) {
+                sc[kt][v] += gd_dpp<GD_DPP_ROR8>(sc[kt][v]);
+                if (lo + 32 * j + 16 * kt + 4 * g + v >= T) sc[kt][v] = -INFINITY;
+                bmax = fmaxf(bmax, sc[kt][v]);
+            }
+        bmax = fmaxf(bmax, __shfl_xor(bmax, 16, 64));
+        bmax = fmaxf(bmax, __shfl_xor(bmax, 32, 64));
+        const float mn = fmaxf(m, bmax);                  // the block's first key is < T
+        if (__any(mn > m)) {
+            const float alpha = __builtin_amdgcn_exp2f(m - mn);
+            l *= alpha;
+#pragma unroll
+            for (int dt = 0; dt < DT; dt++) acc[dt] *= alpha;
+            m = mn;
+        }
+        f16x8 pf;
+#pragma unroll
+        for (int kt = 0; kt < 2; kt++)
+#pragma unroll
+            for (int v = 0; v < 4; v++) {
+                const float p = __builtin_amdgcn_exp2f(sc[kt][v] - m);
+                l += p;
+                f16 hi, lo_;
+                gd_split_f16(p, hi, lo_);
+                pf[4 * kt + v] = lr < 8 ? hi : lo_;
+            }
+        typedef short s16x4 __attribute__((ext_vector_type(4)));
+        typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
+#pragma unroll
+        for (int dt = 0; dt < DT; dt++) {
+            const f16 *vr = &Vs[w][4 * g + (lr >> 2)][16 * dt + 4 * (lr & 3)];
+            const f16x4 v0 = __builtin_bit_cast(f16x4, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4 *)vr));
+            const f16x4 v1 = __builtin_bit_cast(f16x4, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4 *)(vr + 16 * VP)));
+            acc[dt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
+                    f16x8{v0[0], v0[1], v0[2], v0[3], v1[0], v1[1], v1[2], v1[3]}, pf, acc[dt], 0, 0, 0);
+        }
+    }
+    // Merge the waves: each scales its sums to the common maximum.
+    l += __shfl_xor(l, 16, 64);
+    l += __shfl_xor(l, 32, 64);
+    if (lane < 8) {
+        wm[w][lane] = m;
+        wl[w][lane] = l;
+    }
+    __syncthreads();
+    float M = -INFINITY;
+#pragma unroll
+    for (int i = 0; i < PW; i++) M = fmaxf(M, wm[i][c]);
+    const float f = m == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m - M);
+    float *red = (float *)Vs;                             // [PW][8][HD]
+#pragma unroll
+    for (int dt = 0; dt < DT; dt++) {
+#pragma unroll
+        for (int v = 0; v < 4; v++) acc[dt][v] += gd_dpp<GD_DPP_ROR8>(acc[dt][v]);
+        if (lr < 8) *(f32x4 *)&red[(w * 8 + lr) * HD + 16 * dt + 4 * g] = acc[dt] * f;
+    }
+    __syncthreads();
+    for (int e = t; e < nh * HD; e += 64 * PW) {
+        const int hh = e / HD, d = e % HD;
+        float A = 0.f;
+#pragma unroll
+        for (int i = 0; i < PW; i++) A += red[(i * 8 + hh) * HD + d];
+        part[((int64_t)(h0 + hh) * ns + sp) * (HD + 2) + d] = A;
+    }
+    if (t < nh) {
+        float L = 0.f;
+        for (int i = 0; i < PW; i++) L += wm[i][t] == -INFINITY ? 0.f : wl[i][t] * __builtin_amdgcn_exp2f(wm[i][t] - M);
+        float *p = part + ((int64_t)(h0 + t) * ns + sp) * (HD + 2) + HD;
+        p[0] = M;
+        p[1] = L;
+    }
+}
+
 // Merges the DSPLIT partials of head h (HD threads): out[h][d] = A / L,
 // times sigmoid of the raw gate gate[h * gstride + d] when gated.
 template <int HD, typename OT>
@@ -639,6 +810,43 @@ __global__ void k_attn_combine(const float *part, const float *gate, int gstride
     if (gated) o *= gd_sigmoid(gate[(int64_t)h * gstride + t]);
     if constexpr (sizeof(OT) == 2) out[(int64_t)h * HD + t] = gd_f2h(o);
     else out[(int64_t)h * HD + t] = o;
+}
+
+// The same for k_attn_paged's ns <= MAX_SPLITS partials (maxima in units of
+// log2): the splits' weights once per workgroup, then thread (d, r) the
+// splits r, r + NR, .. of one dim, eight loads at a time.
+constexpr int MAX_SPLITS = 64;
+template <int HD>
+__global__ __launch_bounds__(512) void k_attn_paged_combine(const float *part, int ns, const float *gate,
+                                                            int gated, float *out) {
+    constexpr int NR = 512 / HD;
+    __shared__ float fs[MAX_SPLITS], sum[NR][HD];
+    const int h = blockIdx.x, t = threadIdx.x, d = t % HD, r = t / HD;
+    const float *p = part + (int64_t)h * ns * (HD + 2);
+    float inv = 0.f;
+    {
+        const int lane = t & 63;                          // every wave: the weight of split lane
+        const float ms = lane < ns ? p[lane * (HD + 2) + HD] : -INFINITY;
+        const float ls = lane < ns ? p[lane * (HD + 2) + HD + 1] : 0.f;
+        float M = ms;
+        for (int o = 32; o >= 1; o >>= 1) M = fmaxf(M, __shfl_xor(M, o, 64));
+        const float f = ms == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(ms - M);
+        inv = 1.0f / gd_wave_sum(ls * f);
+        if (t < MAX_SPLITS) fs[t] = f;
+    }
+    __syncthreads();
+    float A = 0.f;
+#pragma unroll 8
+    for (int s = r; s < ns; s += NR) A += p[(int64_t)s * (HD + 2) + d] * fs[s];
+    sum[r][d] = A;
+    __syncthreads();
+    if (r == 0) {
+#pragma unroll
+        for (int i = 1; i < NR; i++) A += sum[i][d];
+        float o = A * inv;
+        if (gated) o *= gd_sigmoid(gate[(int64_t)h * HD + d]);
+        out[(int64_t)h * HD + d] = o;
+    }
 }
 
 // ---------------------------------------------------------------- glue
@@ -745,15 +953,15 @@ int gd_attn_decode_launch(gd_ctx *ctx, int hd, const float *proj, int qs, const 
     const float2 *rtab = (const float2 *)rope_tab;
     const int gated = qs == 2 * hd;
     if (hd == 128) {
-        hipLaunchKernelGGL((k_attn_decode<128, true>), grid, dim3(256), 0, ctx->stream, proj, qs,
-                           q_norm, k_norm, kc, vc, page_table, pos_ptr, 0, 0, part, H, HKV, block,
+        hipLaunchKernelGGL((k_attn_decode<128>), grid, dim3(256), 0, ctx->stream, proj, qs,
+                           q_norm, k_norm, kc, vc, page_table, pos_ptr, part, H, HKV, block,
                            scale, n_rot, base, eps, rtab, rope_n);
         GD_LAUNCHED(ctx, "k_attn_decode");
         hipLaunchKernelGGL((k_attn_combine<128, uint16_t>), dim3(H), dim3(128), 0, ctx->stream,
                            part, proj + 128, 2 * 128, gated, out);
     } else {
-        hipLaunchKernelGGL((k_attn_decode<256, true>), grid, dim3(512), 0, ctx->stream, proj, qs,
-                           q_norm, k_norm, kc, vc, page_table, pos_ptr, 0, 0, part, H, HKV, block,
+        hipLaunchKernelGGL((k_attn_decode<256>), grid, dim3(512), 0, ctx->stream, proj, qs,
+                           q_norm, k_norm, kc, vc, page_table, pos_ptr, part, H, HKV, block,
                            scale, n_rot, base, eps, rtab, rope_n);
         GD_LAUNCHED(ctx, "k_attn_decode");
         hipLaunchKernelGGL((k_attn_combine<256, uint16_t>), dim3(H), dim3(256), 0, ctx->stream,
@@ -845,23 +1053,25 @@ extern "C" int gd_attn_paged(gd_ctx *ctx, const float *q, const uint16_t *k_cach
     int rc = check_attn(ctx, "gd_attn_paged", hd, n_head, n_head_kv, kv_dim, page_size, gated, gate);
     if (rc) return rc;
     GD_REQUIRE(ctx, T > 0 && lo >= 0 && lo < T, "gd_attn_paged: keys [lo=%d, T=%d) empty", lo, T);
-    const dim3 grid((unsigned)n_head, DSPLIT);
-    uint16_t *kc = const_cast<uint16_t *>(k_cache), *vc = const_cast<uint16_t *>(v_cache);
-    if (hd == 128) {
-        hipLaunchKernelGGL((k_attn_decode<128, false>), grid, dim3(256), 0, ctx->stream, q,
-                           128, nullptr, nullptr, kc, vc, page_table, nullptr, T, lo, part, n_head,
-                           n_head_kv, page_size, scale, 0, 0.f, 0.f, nullptr, 0);
-        GD_LAUNCHED(ctx, "gd_attn_paged");
-        hipLaunchKernelGGL((k_attn_combine<128, float>), dim3(n_head), dim3(128), 0, ctx->stream,
-                           part, gate, 128, gated, out);
-    } else {
-        hipLaunchKernelGGL((k_attn_decode<256, false>), grid, dim3(512), 0, ctx->stream, q,
-                           256, nullptr, nullptr, kc, vc, page_table, nullptr, T, lo, part, n_head,
-                           n_head_kv, page_size, scale, 0, 0.f, 0.f, nullptr, 0);
-        GD_LAUNCHED(ctx, "gd_attn_paged");
-        hipLaunchKernelGGL((k_attn_combine<256, float>), dim3(n_head), dim3(256), 0, ctx->stream,
-                           part, gate, 256, gated, out);
-    }
+    // Key splits: a block of 32 keys for every wave, up to two workgroups per
+    // CU and what the combine weighs in one wave (64).  More than the 16 a
+    // head that the caller's scratch holds go to the context's own scratch.
+    const int G = n_head / n_head_kv, groups = n_head_kv * ((G + 7) / 8);
+    const int cus = ctx->num_cus > 0 ? ctx->num_cus : 256;
+    const int blocks = (T - lo + 31) / 32;
+    int ns = std::max(1, std::min({(blocks + PW - 1) / PW, MAX_SPLITS, std::max(DSPLIT, 2 * cus / groups)}));
+    if (ns > DSPLIT &&
+        (!ctx->attn_scratch || (size_t)n_head * ns * (hd + 2) * sizeof(float) > GD_ATTN_SCRATCH_BYTES))
+        ns = DSPLIT;
+    float *pt = ns > DSPLIT ? ctx->attn_scratch : part;
+#define GD_PAGED(HD_) \
+    hipLaunchKernelGGL(k_attn_paged<HD_>, dim3(groups, ns), dim3(64 * PW), 0, ctx->stream, q, k_cache, \
+                       v_cache, page_table, T, lo, pt, ns, n_head, n_head_kv, page_size, scale); \
+    GD_LAUNCHED(ctx, "gd_attn_paged"); \
+    hipLaunchKernelGGL(k_attn_paged_combine<HD_>, dim3(n_head), dim3(512), 0, ctx->stream, \
+                       pt, ns, gate, gated, out)
+    if (hd == 128) { GD_PAGED(128); } else { GD_PAGED(256); }
+#undef GD_PAGED
     GD_LAUNCHED(ctx, "gd_attn_paged combine");
     return GD_OK;
 }

@@ -23,8 +23,14 @@ struct gd_ctx {
     // This device's copy of the allocation-free prefill's scratch array
     // (hipGetSymbolAddress at context creation; null if that failed).
     void *prefill_scratch = nullptr;
+    // Key-split partials of gd_attn_paged beyond the 16 per head its caller's
+    // scratch holds: GD_ATTN_SCRATCH_BYTES, held by the context so that the
+    // entry allocates nothing (it may be recorded); null if that failed.
+    float *attn_scratch = nullptr;
     std::string err;
 };
+
+constexpr size_t GD_ATTN_SCRATCH_BYTES = 8u << 20;
 
 // Look up this device's address of the prefill scratch array (device current).
 int gd_prefill_scratch_attach(gd_ctx *ctx);
@@ -254,7 +260,7 @@ template <int CTRL> __device__ __forceinline__ float gd_dpp(float v) {
     return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), CTRL, 0xF, 0xF, false));
 }
 constexpr int GD_DPP_XOR1 = 0xB1, GD_DPP_XOR2 = 0x4E, GD_DPP_HALF_MIRROR = 0x141,
-              GD_DPP_MIRROR = 0x140;
+              GD_DPP_MIRROR = 0x140, GD_DPP_ROR8 = 0x128;   // row rotation by 8: lane i ^ 8
 
 // Sum over each row of 16 lanes, every lane of the row getting it: after the
 // quad exchanges each quad's lanes hold the same value, so the half-row

@@ -65,6 +65,12 @@ extern "C" int gd_ctx_create(int device, gd_ctx **out) {
     // A failed lookup leaves prefill_scratch null: only gd_gdn_prefill_noalloc
     // needs it, and it reports the failure then.
     (void)gd_prefill_scratch_attach(c);
+    // Likewise the attention partials: without them gd_attn_paged splits the
+    // keys no further than its caller's scratch allows.
+    if (hipMalloc((void **)&c->attn_scratch, GD_ATTN_SCRATCH_BYTES) != hipSuccess) {
+        c->attn_scratch = nullptr;
+        (void)hipGetLastError();
+    }
     c->err.clear();
     *out = c;
     return GD_OK;
@@ -77,6 +83,7 @@ extern "C" void gd_ctx_destroy(gd_ctx *ctx) {
     if (ctx->ev_start) (void)hipEventDestroy(ctx->ev_start);
     if (ctx->ev_stop) (void)hipEventDestroy(ctx->ev_stop);
     if (ctx->ws) (void)hipFree(ctx->ws);
+    if (ctx->attn_scratch) (void)hipFree(ctx->attn_scratch);
     if (ctx->stream) (void)hipStreamDestroy(ctx->stream);
     delete ctx;
 }

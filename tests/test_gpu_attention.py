@@ -141,6 +141,29 @@ def test_decode_and_batch_attention(ctx, hd, nh, nkv, page, T):
         ctx.free(p)
 
 
+@pytest.mark.parametrize("hd,nh,nkv,page,T,lo", [
+    (128, 40, 8, 16, 1, 0), (256, 24, 4, 16, 33, 0), (128, 2, 2, 5, 31, 30), (256, 9, 1, 16, 64, 1),
+    (128, 34, 2, 16, 4099, 0), (256, 6, 1, 7, 4097, 100), (128, 16, 8, 16, 9000, 4999)])
+def test_decode_attention_key_blocks(ctx, hd, nh, nkv, page, T, lo):
+    """One query over cached keys lo .. T-1 around the edges of the key blocks
+    and splits (one key, one past a block, several rounds of a wave), with one,
+    two, six and more than eight q heads a kv head: against f64 over the same
+    f16 cache within 3e-6 (22-bit q and weights, f32 sums)."""
+    rng = np.random.default_rng(T + nh)
+    kv_dim, npages = hd * nkv, (T + page - 1) // page + 1
+    table = rng.permutation(npages).astype(np.int32)
+    K, V = (rng.standard_normal((npages, page, nkv, hd)).astype(np.float16) for _ in range(2))
+    q, gate = (rng.standard_normal((nh, hd)).astype(np.float32) for _ in range(2))
+    bufs = [ctx.put(a) for a in (q, K.view(np.uint16), V.view(np.uint16), table, gate)]
+    out, part = ctx.alloc(nh * hd * 4), ctx.alloc(nh * 16 * (hd + 2) * 4)
+    ctx.gd_attn_paged(*bufs, out, part, hd, nh, nkv, T, kv_dim, page, C.c_float(1 / np.sqrt(hd)), 1, lo)
+    rows = lambda a: a[table].reshape(npages * page, nkv, hd)[lo:T]
+    want = ref_attention(q, rows(K), rows(V), gate, nkv, T - lo)
+    assert rel_diff(ctx.get(out, (nh, hd), np.float32), want) < 3e-6
+    for p in (*bufs, out, part):
+        ctx.free(p)
+
+
 def test_attention_rejects_bad_shapes(ctx):
     d = ctx.alloc(64)
     lib = ctx.lib
