@@ -65,6 +65,12 @@ int gd_gemv_mfma_norm(gd_ctx *ctx, const gd_q2w *w, const float *h, const float 
 int gd_gdn_scan_batch_serial(gd_ctx *ctx, const float *convOutN, int keyDim, int valueDim,
                              int convDim, const float *gN, const float *betaN, float *S,
                              float *oN, int nV, int nK, int dS, float qScale, int64_t N);
+// Chunked GDN prefill of f16 q, k, v (gdn_prefill16.hip; arguments checked by
+// the caller as gd_gdn_prefill's) in ws of gd_gdn_prefill16_bytes.
+size_t gd_gdn_prefill16_bytes(int64_t T, int nV, int nK);
+int gd_gdn_prefill16(gd_ctx *ctx, void *ws, int64_t T, int nV, int nK, const void *q, int64_t q_stride,
+                     const void *k, int64_t k_stride, const void *v, int64_t v_stride, const float *g,
+                     const float *beta, float *S, void *o, int64_t o_stride, int o_dtype, float qScale);
 // K splits an f16-x GEMV of this shape should use (partials summed by the consumer).
 int gd_gemv_ksplit(gd_ctx *ctx, int64_t K, int64_t R);
 // Prefill GEMM plan: MT x 32 tokens by 4 x NT x 32 weight rows per
