@@ -77,7 +77,9 @@ int gd_gemv_ksplit(gd_ctx *ctx, int64_t K, int64_t R);
 // workgroup, K split `split` ways into f32 partials.
 // nw: waves per workgroup; ex = 1: the 4 x 2 x 8 tile with a seventeenth
 // 32-row fragment (544 rows a workgroup; f32 out or split partials only).
-struct gd_gemm_plan { int mt, nt, split; int nw = 4; int ex = 0; };
+// skinny = 1: the few-token kernel (T <= 32), K split
+// into `split` runs of 512-K chunks; the tile fields are not used.
+struct gd_gemm_plan { int mt, nt, split; int nw = 4; int ex = 0; int skinny = 0; };
 gd_gemm_plan gd_gemm_choose(gd_ctx *ctx, int64_t T, int64_t K, int64_t R, int x_dtype);
 // split > 1: y_dtype f32 and Y holds split * T * R partials, summed by the caller.
 int gd_gemm_launch(gd_ctx *ctx, const gd_q2w *w, int64_t T, const void *X, int x_dtype, void *Y,

@@ -481,6 +481,165 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(NW == 4
     }
 }
 
+// The GEMM of a few tokens (T <= 32: short prompts, chat turns), where a tile
+// of the kernel above costs each 128-K block two barriers and its waves the
+// issue of every code's direct load.  Here only X goes through LDS, in chunks
+// of 512 K (two stages, one barrier a chunk); a wave takes its codes (16 bytes
+// a lane and block, one contiguous KiB) and scales straight into registers, two
+// chunks ahead.  Wave (f, kp) of the 8 multiplies all tokens by the 32 rows of
+// fragment f (of 2) at block kp (of 4) of every chunk, on two accumulator
+// chains (even and odd K-steps); the four parts are summed through LDS at the
+// end.  K order inside a block: lane half lh, step s, element e carry K = 64 lh
+// + 8 s + e, so a lane's 16 code bytes are its block half.
+// Bound by what one CU takes in, 40 KiB of X and codes in 0.65 us a chunk and
+// workgroup (0.3 us without the loads, 0.67 without the arithmetic): each 64
+// rows read all of X again.  Rings of 3 and 4 stages, 4 fragments x 2 blocks,
+// 16 waves, other chunk orders and 64 tokens a wave were no faster.
+// nz > 1: K split z takes chunks z cps .. and writes f32 partials at Y + z T R.
+// glu_ff > 0 (nz = 1): fragments of 16 gate and their 16 up rows, f16 SwiGLU
+// output as above.
+constexpr int SK_K = 512, SK_WAVES = 8, SK_FRAGS = 2;   // K per chunk (a step of the code tiles)
+__global__ __launch_bounds__(64 * SK_WAVES) __attribute__((amdgpu_waves_per_eu(4))) void q2_0_gemm_skinny(
+        const uint8_t *codes, const uint16_t *scales, const uint16_t *X, void *Y, int y16, int T, int K, int R, int nfrag,
+        int cps, int glu_ff) {
+    constexpr int ROWB = SK_K * 2, STAGE = 32 * ROWB;
+    extern __shared__ __attribute__((aligned(16))) uint8_t lds[];   // [2][32][SK_K] f16, swizzled
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int f = wave >> 2, kp = wave & 3;
+    const int li = lane & 31, lh = lane >> 5;
+    const int frag = (int)blockIdx.x * SK_FRAGS + f, z = (int)blockIdx.y;
+    const int nblk = K >> 7, csteps = (nblk + 3) >> 2, bgroups = (nblk + 15) >> 4;
+    const int c_begin = z * cps, c_end = min(c_begin + cps, csteps);
+    // Codes and scales of the fragment's row groups: 2 frag and 2 frag + 1
+    // (lanes 16..31 of a half), with SwiGLU gate group frag and up group glu_ff /
+    // 16 + frag.  Groups past R lie beyond the resources and load as zeros.
+    const int g0 = glu_ff ? frag : 2 * frag, rgroups = (R + 15) >> 4;
+    const uint32_t gvalid = (uint32_t)max(0, min(glu_ff ? (glu_ff >> 4) + 1 : 2, rgroups - g0));
+    const __amdgpu_buffer_rsrc_t crs =
+            gd_rsrc(codes + ((size_t)g0 * csteps << 11), gvalid * (uint32_t)csteps * 2048u);
+    const __amdgpu_buffer_rsrc_t srs =
+            gd_rsrc(scales + (size_t)g0 * bgroups * 256, gvalid * (uint32_t)bgroups * 512u);
+    const uint32_t up = (li >> 4) ? (glu_ff ? (uint32_t)glu_ff >> 4 : 1u) : 0u;
+    const uint32_t cvo = ((up * csteps) << 11) + ((uint32_t)lh << 10) + ((li & 15) << 4);
+    const uint32_t svo = (up * bgroups * 256 + (li & 15)) * 2;
+    // The wave's block of chunk c; past the end of K the last block's codes
+    // (used with scale zero, or not at all).
+    u32x4 cw[2];
+    uint16_t sc[2];
+    auto fetch = [&](int c, int slot) {
+        const int b = min(4 * c + kp, nblk - 1);
+        cw[slot] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(
+                crs, cvo, ((uint32_t)(b >> 2) << 11) + ((uint32_t)(b & 3) << 8), 0));
+        sc[slot] = (uint16_t)__builtin_amdgcn_raw_buffer_load_b16(
+                srs, svo, (uint32_t)((b >> 4) * 256 + (b & 15) * 16) * 2, 0);
+    };
+    // X chunk c into stage st: one row (1 KiB) a load, rows wave, wave + 8 ..;
+    // lane l brings 16-byte piece l ^ (row & 15), so that the 16 rows a b128
+    // read serves together lie on distinct banks.  Tokens past T, what lies past
+    // K and chunks past the split's end get offsets beyond the resource: zeros.
+    // No branch stands between these loads and those of the codes, so that the
+    // compiler's own waits stay exact.
+    const __amdgpu_buffer_rsrc_t xrs = gd_rsrc(X, (uint32_t)T * K * 2);
+    auto stage_x = [&](int c, int st) {
+#pragma unroll
+        for (int i = 0; i < 32 / SK_WAVES; i++) {
+            const int r = wave + SK_WAVES * i, piece = lane ^ (r & 15);
+            const bool in = c < c_end && c * SK_K + 8 * piece < K;
+            lds_load16(xrs, lds + st * STAGE + r * ROWB,
+                       in ? (uint32_t)r * K * 2 + (uint32_t)c * ROWB + (piece << 4) : 0x80000000u, 0);
+        }
+    };
+    f32x16 acc[2];
+#pragma unroll
+    for (int a = 0; a < 2; a++)
+#pragma unroll
+        for (int v = 0; v < 16; v++) acc[a][v] = 0.f;
+    // Chunk c in stage (and register slot) h: its direct loads are older than
+    // the codes and scale requested in the chunk before it, all that may still
+    // be outstanding; the barrier also ends every wave's reads of the other
+    // stage, which the next chunk's loads then fill.  The fences (and pointers
+    // without __restrict__, past whose reads the waits may not move) keep that
+    // order of requests.
+    auto chunk = [&](int c, auto half) {
+        constexpr int h = decltype(half)::value;
+        __builtin_amdgcn_sched_barrier(0);
+        asm volatile("s_waitcnt vmcnt(2) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        stage_x(c + 1, h ^ 1);
+        __builtin_amdgcn_sched_barrier(0);
+        const uint8_t *xb = lds + h * STAGE + li * ROWB;
+        const u32x4 w4 = cw[h];
+        const f16 d = 4 * c + kp < nblk ? __builtin_bit_cast(f16, sc[h]) : (f16)0.f;
+        const f16x2 d2 = {d, d}, nd2 = -d2;
+#pragma unroll
+        for (int s = 0; s < 8; s++) {
+            const uint32_t w = w4[s >> 1];
+            const f16x8 b = dequant8((s & 1 ? w >> 2 : w) & 0x33333333u, d2, nd2);
+            const f16x8 a = *(const f16x8 *)(xb + (((16 * kp + 8 * lh + s) ^ (li & 15)) << 4));
+            acc[s & 1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, acc[s & 1], 0, 0, 0);
+        }
+        fetch(c + 2, h);
+    };
+    stage_x(c_begin, 0);
+    __builtin_amdgcn_sched_barrier(0);
+    fetch(c_begin, 0);
+    __builtin_amdgcn_sched_barrier(0);
+    fetch(c_begin + 1, 1);
+    for (int c = c_begin;;) {
+        chunk(c, std::integral_constant<int, 0>{});
+        if (++c >= c_end) break;
+        chunk(c, std::integral_constant<int, 1>{});
+        if (++c >= c_end) break;
+    }
+    f32x16 sum = acc[0] + acc[1];
+    // Sum the four parts (the stages are free once every wave is past its loop).
+    float *red = (float *)lds;                            // [SK_FRAGS][3][16][64]
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    if (kp) {
+#pragma unroll
+        for (int v = 0; v < 16; v++) red[((f * 3 + kp - 1) * 16 + v) * 64 + lane] = sum[v];
+    }
+    __syncthreads();
+    if (kp || frag >= nfrag) return;
+#pragma unroll
+    for (int p = 0; p < 3; p++)
+#pragma unroll
+        for (int v = 0; v < 16; v++) sum[v] += red[((f * 3 + p) * 16 + v) * 64 + lane];
+    // Lane column li = weight row, accumulator rows 8 (v / 4) + 4 lh + v % 4 =
+    // tokens (those past T lie beyond the output's resource: not stored).
+    const uint32_t ybytes = (uint32_t)T * (glu_ff ? glu_ff : R) * (glu_ff || y16 ? 2u : 4u);
+    const __amdgpu_buffer_rsrc_t yrs = gd_rsrc((uint8_t *)Y + (size_t)z * ybytes, ybytes);
+    if (glu_ff) {
+        const bool gl = li < 16;
+        const uint32_t o0 = (uint32_t)(4 * lh + (gl ? 0 : 16)) * glu_ff + 16 * frag + (li & 15);
+#pragma unroll
+        for (int q = 0; q < 8; q++) {
+            const float lo = sum[q], hi = sum[8 + q];
+            const float other = __shfl_xor(gl ? hi : lo, 16, 64);
+            const float mine = gl ? lo : hi;
+            const float gate = gl ? mine : other, upv = gl ? other : mine;
+            const float sg = gate * __builtin_amdgcn_rcpf(1.0f + __expf(-gate));
+            __builtin_amdgcn_raw_buffer_store_b16(gd_f2h(sg * upv), yrs,
+                                                  (o0 + (uint32_t)(8 * (q >> 2) + (q & 3)) * glu_ff) * 2, 0, 0);
+        }
+        return;
+    }
+    const int r = 32 * frag + li;
+    if (r >= R) return;
+    const uint32_t y0 = (uint32_t)(4 * lh) * R + r;
+    if (y16) {
+#pragma unroll
+        for (int v = 0; v < 16; v++)
+            __builtin_amdgcn_raw_buffer_store_b16(gd_f2h(sum[v]), yrs,
+                                                  (y0 + (uint32_t)(8 * (v >> 2) + (v & 3)) * R) * 2, 0, 0);
+    } else {
+#pragma unroll
+        for (int v = 0; v < 16; v++)
+            __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(sum[v]), yrs,
+                                                  (y0 + (uint32_t)(8 * (v >> 2) + (v & 3)) * R) * 4, 0, 0);
+    }
+}
+
 // Y[i] = sum_z P[z][i] (n elements, 4 per thread).
 template <int YT>
 __global__ __launch_bounds__(256) void q2_0_gemm_reduce(const float *__restrict__ P,
@@ -598,6 +757,14 @@ double round_cost(const Shape &sh, int64_t units, int cus, int bps) {
 //   * split partials cost (2s+1) f32 passes over T x R (CS us per MB).
 // The plan depends on the shape and the CU count alone (no process-wide
 // override); gd_q2_0_gemm_plan runs a plan the caller chooses.
+// At most 32 tokens go to q2_0_gemm_skinny as long as its workgroups (64 rows)
+// take one round of the CUs: 16 x 5120 x 8224 11.8 -> 9.0 us, 27 x 17408 x
+// 5120 18.4 -> 15.0, 32 x 5120 x 5120 10.7 -> 8.5, 8 x 2048 x 5120 6.9 -> 5.4,
+// 32 x 12288 x 12288 21.7 -> 20.4, 32 x 512 x 512 5.9 -> 3.6.  In a second
+// round the tiles draw level (27 x 5120 x 17408: 16.6, skinny 17.3) and ahead
+// (20 x 5120 x 98304: 51.2, skinny 52.7; 3 x 128 x 70000: 3.6, skinny 9.2).
+// Its K is split while the splits fit the round and save more chunks, at
+// 0.65 us each, than the reduction's launch and traffic cost.
 gd_gemm_plan gd_gemm_choose(gd_ctx *ctx, int64_t T, int64_t K, int64_t R, int x_dtype) {
     (void)x_dtype;
     const int nblk = (int)(K / 128);
@@ -606,6 +773,22 @@ gd_gemm_plan gd_gemm_choose(gd_ctx *ctx, int64_t T, int64_t K, int64_t R, int x_
         return (nblk + bps - 1) / bps;
     };
     const int cus = ctx->num_cus > 0 ? ctx->num_cus : 256;
+    const int64_t skinny_wgs = (R + 32 * SK_FRAGS - 1) / (32 * SK_FRAGS);
+    if (T <= 32 && skinny_wgs <= cus) {
+        const int chunks = (int)((K + SK_K - 1) / SK_K);
+        gd_gemm_plan best{1, 1, 1, 4, 0, 1};
+        double best_cost = 1e30;
+        for (int s = 1; s <= 8 && s * skinny_wgs <= cus; s++) {
+            const int cps = (chunks + s - 1) / s;
+            if ((chunks + cps - 1) / cps < s) continue;   // the same as a smaller split
+            const double cost = 0.65 * cps + (s > 1 ? 2.0 + CS * (2.0 * s + 1) * (double)T * R * 4 / 1e6 : 0.0);
+            if (cost < best_cost) {
+                best_cost = cost;
+                best.split = s;
+            }
+        }
+        return best;
+    }
     // Measured plans for the config-4 stack's prefill shapes and the 17408-row
     // gate|up at T = 512 on a full MI355X (the fastest of 29-41 forced plans,
     // min of repeated sweeps); the cost model below mispredicts the 2 x 1 x 4
@@ -645,12 +828,30 @@ gd_gemm_plan gd_gemm_choose(gd_ctx *ctx, int64_t T, int64_t K, int64_t R, int x_
     return best;
 }
 
+// Launch of the few-token kernel over nfrag fragments (32 rows, or 16 gate and
+// 16 up ones with glu_ff), K split into nz.
+static int launch_skinny(gd_ctx *ctx, const gd_q2w *w, int64_t T, const void *X, void *Y, int y16,
+                         int nfrag, int nz, int glu_ff) {
+    const int chunks = gd_blocks(w->K, SK_K), cps = (chunks + nz - 1) / nz;
+    hipLaunchKernelGGL(q2_0_gemm_skinny, dim3(gd_blocks(nfrag, SK_FRAGS), (unsigned)gd_blocks(chunks, cps)),
+                       dim3(64 * SK_WAVES), 2 * 32 * SK_K * 2, ctx->stream, (const uint8_t *)w->codes,
+                       (const uint16_t *)w->scales, (const uint16_t *)X, Y, y16, (int)T, (int)w->K,
+                       (int)w->R, nfrag, cps, glu_ff);
+    GD_LAUNCHED(ctx, "q2_0_gemm_skinny");
+    return GD_OK;
+}
+
 // Launch one plan on f16 X.  plan.split > 1 requires y_dtype f32 and Y sized
 // split * T * R (partials, summed by the caller).
 int gd_gemm_launch(gd_ctx *ctx, const gd_q2w *w, int64_t T, const void *X, int x_dtype, void *Y,
                    int y_dtype, const gd_gemm_plan &p) {
     const int K = (int)w->K, R = (int)w->R;
     const int nblk = K / 128;
+    if (p.skinny) {
+        GD_REQUIRE(ctx, T <= 32 && x_dtype == GD_F16 && (p.split == 1 || y_dtype == GD_F32) && R < (1 << 22),
+                   "gd_q2_0_gemm: bad few-token plan");
+        return launch_skinny(ctx, w, T, X, Y, p.split == 1 && y_dtype == GD_F16, (R + 31) / 32, p.split, 0);
+    }
     const int bps = (nblk + p.split - 1) / p.split;     // blocks (128 K) per split
     const int nz = (nblk + bps - 1) / bps;
     const int yt = p.split > 1 ? 0 : (y_dtype == GD_F16);
@@ -718,6 +919,10 @@ int gd_gemm_glu(gd_ctx *ctx, const gd_q2w *w, int64_t T, const void *X, uint16_t
     GD_REQUIRE(ctx, (uint64_t)(R / 32 + 2) * (uint64_t)((nblk + 3) / 4) * 2048u < (1ULL << 32),
                "gd_gemm_glu: K=%d R=%d spans 4 GiB of codes in one buffer resource", K, R);
     const int cus = ctx->num_cus > 0 ? ctx->num_cus : 256;
+    // Few tokens: 27 x 5120, ff 17408 34.5 -> 26.8 us (weights from HBM), 16 x
+    // 4096, ff 12288 18.6 -> 12.8, 32 x 2048, ff 6144 10.8 -> 6.0, 7 x 384, ff
+    // 48 4.5 -> 4.2.  A forced tile plan stays with the tiles.
+    if (T <= 32 && tile17 < 0) return launch_skinny(ctx, w, T, X, out, 1, ff / 16, 1, ff);
     auto cols = [](const Shape &sh) { return 16 * sh.nw * sh.nt; };
     auto tiles_t = [&](const Shape &sh) { return (T + sh.mt * 32 - 1) / (sh.mt * 32); };
     // One launch of tile sh over ncols columns, K split into nz parts (the
@@ -827,7 +1032,7 @@ int gemm_run(gd_ctx *ctx, const gd_q2w *w, int64_t T, const void *X, int x_dtype
                    "gd_q2_0_gemm_plan: no kernel for mt=%d nt=%d split=%d nw=%d", forced->mt,
                    forced->nt, forced->split, forced->nw);
         p = *forced;
-        const int nblk = (int)(w->K / 128);
+        const int nblk = p.skinny ? (int)(w->K / 128 + 3) / 4 : (int)(w->K / 128);
         const int bps = (nblk + p.split - 1) / p.split;
         p.split = (nblk + bps - 1) / bps;               // splits that hold blocks
     } else {
@@ -880,7 +1085,7 @@ extern "C" int gd_q2_0_gemm(gd_ctx *ctx, const gd_q2w *w, int64_t T, const void 
 extern "C" int gd_q2_0_gemm_plan(gd_ctx *ctx, const gd_q2w *w, int64_t T, const void *X,
                                  int x_dtype, void *Y, int y_dtype, int mt, int nt, int split,
                                  int nw) {
-    const gd_gemm_plan p{mt, nt, split, nw};
+    gd_gemm_plan p{mt, nt, split, nw};
     return gemm_run(ctx, w, T, X, x_dtype, Y, y_dtype, &p);
 }
 

@@ -757,7 +757,7 @@ int forward(gd_stack *st, int N, bool decode) {
                 R_(gd_gemm_launch(ctx, &ly.in_proj, N, st->xn16, GD_F16, st->contrib, GD_F32, pi));
                 pin = st->contrib;
                 np = pi.split;
-            } else if (pi.split == 1 && !pi.ex && r0 < ly.in_proj.R && r0 >= off_b && TAIL_SPLITS <= TAIL_MAX &&
+            } else if (pi.split == 1 && !pi.ex && !pi.skinny && r0 < ly.in_proj.R && r0 >= off_b && TAIL_SPLITS <= TAIL_MAX &&
                        (size_t)TAIL_SPLITS * N * (ly.in_proj.R - r0) <= (size_t)8 * st->c.max_batch * E) {
                 tail_np = TAIL_SPLITS;
                 R_(gd_gemm_launch_tail(ctx, &ly.in_proj, N, st->xn16, st->proj, pi, st->contrib,
