@@ -13,15 +13,15 @@
 // which is how a HIP caller would lay pages out.
 //
 // MI355X design:
-//   * Decode (one query), gd_attn_paged: flash decoding on the matrix cores,
-//     a kv head's keys read once for all its q heads (k_attn_paged).
-//   * Decode, the stack's variant (k_attn_decode): flash decoding, DSPLIT key
+//   * Decode (one query), many keys, gd_attn_paged: flash decoding on the matrix
+//     cores, a kv head's keys read once for all its q heads (k_attn_paged).
+//   * Decode, few keys and the stack (k_attn_decode): flash decoding, DSPLIT key
 //     splits per head; each wave takes whole keys, a lane holding HD/64
 //     consecutive dims, with an online softmax; a block merges its waves and
 //     writes (max, sum, acc[HD]); a combine kernel merges the splits with the
-//     output gate.  It folds in the per-token preparation (split of q|gate,
-//     RMS norm, partial NEOX rope, the cache append), so the new key never
-//     round-trips through the cache within the step.
+//     output gate.  The stack's variant folds in the per-token preparation
+//     (split of q|gate, RMS norm, partial NEOX rope, the cache append), so the
+//     new key never round-trips through the cache within the step.
 //   * Prefill (N queries): flash attention on the matrix cores, block (head,
 //     64 queries); keys in blocks of 64 (32 for head dim 256) through LDS,
 //     K and V as stored, V^T taken by the transposing LDS read; S^T = K Q^T
@@ -417,24 +417,27 @@ __global__ __launch_bounds__(256) void k_attn_prefill(
 
 // ---------------------------------------------------------------- decode
 
-// The stack's decode attention for one query token, split over keys (flash
-// decoding): block (head h, split sp) of 2 HD threads (NWD = HD / 32 waves).
-// The block prepares its own q from the projection row (q of head h at h qs:
-// the q half of a [q | gate] pair when qs = 2 HD, plain q when qs = HD; RMS
-// norm, rope; threads 0..HD-1) and the new k and v (threads HD..2HD-1),
-// rounded to f16 as the cache stores them; the split that holds key pos uses
-// them for that key instead of reading the cache, and the first q head of
-// each kv group appends them.  No block reads the cache at pos.
-// Each wave takes whole keys j = NWD sp + w + STEP i with a lane holding
+// Decode attention for one query token, split over keys (flash decoding):
+// block (head h, split sp) of 2 HD threads (NWD = HD / 32 waves).
+//   FUSED (the stack): the block prepares its own q from the projection row
+//   (q of head h at h qs: the q half of a [q | gate] pair when qs = 2 HD,
+//   plain q when qs = HD; RMS norm, rope; threads 0..HD-1) and the
+//   new k and v (threads HD..2HD-1), rounded to f16 as the cache stores them;
+//   the split that holds key pos uses them for that key instead of reading
+//   the cache, and the first q head of each kv group appends them.  No block
+//   reads the cache at pos.
+//   Otherwise (gd_attn_paged): q arrives prepared, the T keys lo .. T-1 are
+//   all cached.
+// Each wave takes whole keys j = lo + NWD sp + w + STEP i with a lane holding
 // HD/64 consecutive dims, keeping an online-softmax partial; the block
 // merges its waves and writes (max, sum, acc[HD]) for the split; the combine
 // kernel merges the splits (Attention.swift:108-134).  A wave keeps the K
 // and V of its next KB keys in flight (a register ring), their page-table
 // entries one round ahead of them, so a key waits for neither.
-template <int HD>
+template <int HD, bool FUSED>
 __global__ __launch_bounds__(2 * HD) void k_attn_decode(
         const float *src, int qs, const float *q_norm, const float *k_norm, uint16_t *kc,
-        uint16_t *vc, const int32_t *page_table, const int32_t *pos_ptr, float *part,
+        uint16_t *vc, const int32_t *page_table, const int32_t *pos_ptr, int T, int lo, float *part,
         int H, int HKV, int block, float scale, int n_rot, float base, float eps,
         const float2 *rtab, int rtab_n) {
     constexpr int NT = 2 * HD, NWD = NT / 64, DPL = HD / 64, WPH = HD / 64;
@@ -445,9 +448,10 @@ __global__ __launch_bounds__(2 * HD) void k_attn_decode(
     const int h = blockIdx.x, sp = blockIdx.y, t = threadIdx.x;
     const int lane = t & 63, w = __builtin_amdgcn_readfirstlane(t >> 6);
     const int kvh = h / (H / HKV), kvDim = HKV * HD;
-    // Keys read from the cache: [0, pos), pos the new token's position.
-    const int pos = *pos_ptr;
-    const bool has_pos = sp == (pos / NWD) % DSPLIT;   // wave pos % NWD takes key pos
+    // Keys read from the cache: [lo, pos) for the stack (pos = the new
+    // token's position, taken from its registers), [lo, T) otherwise.
+    const int pos = FUSED ? *pos_ptr : T;
+    const bool has_pos = FUSED && sp == (pos / NWD) % DSPLIT;   // wave pos % NWD takes key pos
     // A lane's DPL f16 dims of one key: one dword (HD 128) or two (HD 256).
     using U = typename std::conditional<DPL == 2, uint32_t, u32x2>::type;
     auto ld = [&](const uint16_t *p) { return *(const U *)p; };
@@ -457,13 +461,14 @@ __global__ __launch_bounds__(2 * HD) void k_attn_decode(
     };
     // Cached keys of this wave: j0 + STEP i, i < nk.  Every load below is
     // unconditional (the compiler waits exactly only for straight-line
-    // loads): a key past the last reads position pos instead, whose page
-    // exists (the new token's), and is not used.
-    const int j0 = sp * NWD + w;
+    // loads): a key past the last reads position jlast instead, whose page
+    // exists (the new token's, or the last cached key's), and is not used.
+    const int j0 = lo + sp * NWD + w;
     const int nk = j0 < pos ? (pos - 1 - j0) / STEP + 1 : 0;
+    const int jlast = FUSED ? pos : T - 1;
     auto kpos = [&](int i) {
         const int jj = j0 + i * STEP;
-        return jj < pos ? jj : pos;
+        return jj < pos ? jj : jlast;
     };
     // Cache slots of keys i0 .. i0 + KB - 1, lane l holding key i0 + l % KB:
     // its page-table entry (a load) and its position in the page.
@@ -497,7 +502,7 @@ __global__ __launch_bounds__(2 * HD) void k_attn_decode(
         pg = entries(KB);
         __builtin_amdgcn_sched_barrier(0);
     };
-    {
+    if constexpr (FUSED) {
         // q of head h (hf = 0) and k of kv head kvh (hf = 1): RMS norm over
         // the head, then the partial NEOX rope, as k_attn_prep.
         const int H2 = H * qs;
@@ -537,6 +542,11 @@ __global__ __launch_bounds__(2 * HD) void k_attn_decode(
             kc[slot * kvDim + kvh * HD + i] = gd_f2h(y);
             vc[slot * kvDim + kvh * HD + i] = gd_f2h(vnew[i]);
         }
+    } else {
+        const float qx = t < HD ? src[(int64_t)h * HD + t] : 0.f;
+        prime();
+        if (t < HD) rot[0][t] = qx;
+        __syncthreads();
     }
     float qv[DPL], a[DPL];
 #pragma unroll
@@ -574,7 +584,7 @@ __global__ __launch_bounds__(2 * HD) void k_attn_decode(
 #pragma unroll
     for (int s = 0; s < KB; s++)
         if (i + s < nk) consume(kr[s], vr[s]);
-    {
+    if constexpr (FUSED) {
         // Key pos, from this block's own copy (f16, as cached).
         if (has_pos && w == pos % NWD) {
             uint32_t kw[DPL / 2], vw[DPL / 2];
@@ -621,13 +631,17 @@ __global__ __launch_bounds__(2 * HD) void k_attn_decode(
 // barrier in the loop).  The 16 columns of an MFMA are the eight heads' q as
 // f16 hi (columns 0..7) and lo (8..15), and P likewise, so both halves of a
 // product come from one instruction and are added across lanes lr, lr ^ 8.
-// Scores are in units of log2 (q is scaled by scale log2 e).  A block's K and
+// Scores are in units of log2 (times scale log2 e).  A block's K and
 // V are requested one block ahead, its page-table entries two.
 //   Bound by the latency of a few rounds of loads: one wave a key and q head,
 // with a wave reduction per key, took 42 us at 9001 keys of 24 / 4 heads x 256
 // (37 MB, each read by six heads' workgroups); this, on the 16 splits of
 // eight waves that the caller's scratch allows, 21 us (64 CUs), on 64 splits of
 // four 13; 32000 keys 27 us (4.9 TB/s of cache).
+//   Against 64 bits (24 / 4 x 256, unit normal q, K, V): 2.1e-7 of the output at
+// 3000 and at 9001 keys, 2.2e-7 at 30000; one wave a key in f32 1.8e-7,
+// 2.2e-7, 3.2e-7.  With unscaled q and weights the low halves fell below
+// f16's normal range (3.4e-7).
 constexpr int PW = 4;           // waves
 constexpr float LOG2E = 1.4426950408889634f;
 template <int HD>
@@ -672,19 +686,39 @@ __global__ __launch_bounds__(64 * PW) __attribute__((amdgpu_waves_per_eu(2, 2)))
     int j = sp + ns * w;
     int sl = slot_of(j), sn = slot_of(j + step);
     // Q's operand, once per workgroup (it does not fit the registers beside
-    // a block of K and V and the sums at head dim 256).
-    for (int ks = w; ks < KS; ks += PW) {
-        const float *qrow = q + (int64_t)(h0 + min(c, nh - 1)) * HD + 32 * ks + 8 * g;
-        const f32x4 a = *(const f32x4 *)qrow, b = *(const f32x4 *)(qrow + 4);
-        const float qs = c < nh ? scale * LOG2E : 0.f;
-        f16x8 qf;
+    // a block of K and V and the sums at head dim 256): each head's q times the
+    // power of two that brings its largest into 2^14 .. 2^15, so that neither
+    // half of the split leaves f16's normal range, whatever q's size.
+    float sf;                                             // score factor of head c
+    {
+        const float *qrow = q + (int64_t)(h0 + min(c, nh - 1)) * HD + 8 * g;
+        f32x4 qv[KS][2];
+        float mx = 0.f;
 #pragma unroll
-        for (int e = 0; e < 8; e++) {
-            f16 hi, lo_;
-            gd_split_f16((e < 4 ? a[e] : b[e - 4]) * qs, hi, lo_);
-            qf[e] = lr < 8 ? hi : lo_;
+        for (int ks = 0; ks < KS; ks++)
+#pragma unroll
+            for (int e = 0; e < 2; e++) {
+                qv[ks][e] = *(const f32x4 *)(qrow + 32 * ks + 4 * e);
+#pragma unroll
+                for (int i = 0; i < 4; i++) mx = fmaxf(mx, fabsf(qv[ks][e][i]));
+            }
+        mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
+        mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+        const int ex = min(max((int)(__float_as_uint(mx) >> 23), 40), 254) - 127;
+        const float up = __uint_as_float((uint32_t)(127 + 14 - ex) << 23);
+        sf = scale * LOG2E * __uint_as_float((uint32_t)(127 - 14 + ex) << 23);
+#pragma unroll
+        for (int ks = 0; ks < KS; ks++) {
+            if (ks % PW != w) continue;
+            f16x8 qf;
+#pragma unroll
+            for (int e = 0; e < 8; e++) {
+                f16 hi, lo_;
+                gd_split_f16(c < nh ? qv[ks][e >> 2][e & 3] * up : 0.f, hi, lo_);
+                qf[e] = lr < 8 ? hi : lo_;
+            }
+            Qs[ks][lane] = qf;
         }
-        Qs[ks][lane] = qf;
     }
     fetchK(sl);
     fetchV(sl);
@@ -694,15 +728,21 @@ __global__ __launch_bounds__(64 * PW) __attribute__((amdgpu_waves_per_eu(2, 2)))
     float m = -INFINITY, l = 0.f;                         // l: this lane's keys only
     __syncthreads();
     for (; j < nb; j += step) {
-        f32x4 sc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+        // Four chains a key tile: shorter sums round less (and wait less).
+        f32x4 st[2][4];
 #pragma unroll
         for (int ks = 0; ks < KS; ks++) {
             const f16x8 qf = Qs[ks][lane];
 #pragma unroll
             for (int kt = 0; kt < 2; kt++)
-                sc[kt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, kreg[kt][ks]), qf, sc[kt],
-                                                                0, 0, 0);
+                st[kt][ks & 3] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
+                        __builtin_bit_cast(f16x8, kreg[kt][ks]), qf,
+                        ks < 4 ? f32x4{0.f, 0.f, 0.f, 0.f} : st[kt][ks & 3], 0, 0, 0);
         }
+        f32x4 sc[2];
+#pragma unroll
+        for (int kt = 0; kt < 2; kt++)
+            sc[kt] = (st[kt][0] + st[kt][1]) + (st[kt][2] + st[kt][3]);
         __builtin_amdgcn_sched_barrier(0);
         const int s2 = slot_of(j + 2 * step);
         fetchK(sn);
@@ -718,7 +758,7 @@ __global__ __launch_bounds__(64 * PW) __attribute__((amdgpu_waves_per_eu(2, 2)))
         for (int kt = 0; kt < 2; kt++)
 #pragma unroll
             for (int v = 0; v < 4; v++) {
-                sc[kt][v] += gd_dpp<GD_DPP_ROR8>(sc[kt][v]);
+                sc[kt][v] = (sc[kt][v] + gd_dpp<GD_DPP_ROR8>(sc[kt][v])) * sf;
                 if (lo + 32 * j + 16 * kt + 4 * g + v >= T) sc[kt][v] = -INFINITY;
                 bmax = fmaxf(bmax, sc[kt][v]);
             }
@@ -732,12 +772,14 @@ __global__ __launch_bounds__(64 * PW) __attribute__((amdgpu_waves_per_eu(2, 2)))
             for (int dt = 0; dt < DT; dt++) acc[dt] *= alpha;
             m = mn;
         }
+        // Weights times 2^14 (so are l and the sums): small ones keep their lo
+        // (in the exponent the 14 would round the score).
         f16x8 pf;
 #pragma unroll
         for (int kt = 0; kt < 2; kt++)
 #pragma unroll
             for (int v = 0; v < 4; v++) {
-                const float p = __builtin_amdgcn_exp2f(sc[kt][v] - m);
+                const float p = __builtin_amdgcn_exp2f(sc[kt][v] - m) * 16384.f;
                 l += p;
                 f16 hi, lo_;
                 gd_split_f16(p, hi, lo_);
@@ -813,8 +855,8 @@ __global__ void k_attn_combine(const float *part, const float *gate, int gstride
 }
 
 // The same for k_attn_paged's ns <= MAX_SPLITS partials (maxima in units of
-// log2): the splits' weights once per workgroup, then thread (d, r) the
-// splits r, r + NR, .. of one dim, eight loads at a time.
+// log2): thread (d, r) takes the splits r, r + NR, .. of one dim, all requested
+// at once, beside the splits' weights, once per workgroup.
 constexpr int MAX_SPLITS = 64;
 template <int HD>
 __global__ __launch_bounds__(512) void k_attn_paged_combine(const float *part, int ns, const float *gate,
@@ -823,6 +865,10 @@ __global__ __launch_bounds__(512) void k_attn_paged_combine(const float *part, i
     __shared__ float fs[MAX_SPLITS], sum[NR][HD];
     const int h = blockIdx.x, t = threadIdx.x, d = t % HD, r = t / HD;
     const float *p = part + (int64_t)h * ns * (HD + 2);
+    // Past the last split: the last one, at weight zero.
+    float a[MAX_SPLITS / NR];
+#pragma unroll
+    for (int s = 0; s < MAX_SPLITS / NR; s++) a[s] = p[(int64_t)min(r + NR * s, ns - 1) * (HD + 2) + d];
     float inv = 0.f;
     {
         const int lane = t & 63;                          // every wave: the weight of split lane
@@ -836,8 +882,8 @@ __global__ __launch_bounds__(512) void k_attn_paged_combine(const float *part, i
     }
     __syncthreads();
     float A = 0.f;
-#pragma unroll 8
-    for (int s = r; s < ns; s += NR) A += p[(int64_t)s * (HD + 2) + d] * fs[s];
+#pragma unroll
+    for (int s = 0; s < MAX_SPLITS / NR; s++) A += a[s] * fs[r + NR * s];
     sum[r][d] = A;
     __syncthreads();
     if (r == 0) {
@@ -953,15 +999,15 @@ int gd_attn_decode_launch(gd_ctx *ctx, int hd, const float *proj, int qs, const 
     const float2 *rtab = (const float2 *)rope_tab;
     const int gated = qs == 2 * hd;
     if (hd == 128) {
-        hipLaunchKernelGGL((k_attn_decode<128>), grid, dim3(256), 0, ctx->stream, proj, qs,
-                           q_norm, k_norm, kc, vc, page_table, pos_ptr, part, H, HKV, block,
+        hipLaunchKernelGGL((k_attn_decode<128, true>), grid, dim3(256), 0, ctx->stream, proj, qs,
+                           q_norm, k_norm, kc, vc, page_table, pos_ptr, 0, 0, part, H, HKV, block,
                            scale, n_rot, base, eps, rtab, rope_n);
         GD_LAUNCHED(ctx, "k_attn_decode");
         hipLaunchKernelGGL((k_attn_combine<128, uint16_t>), dim3(H), dim3(128), 0, ctx->stream,
                            part, proj + 128, 2 * 128, gated, out);
     } else {
-        hipLaunchKernelGGL((k_attn_decode<256>), grid, dim3(512), 0, ctx->stream, proj, qs,
-                           q_norm, k_norm, kc, vc, page_table, pos_ptr, part, H, HKV, block,
+        hipLaunchKernelGGL((k_attn_decode<256, true>), grid, dim3(512), 0, ctx->stream, proj, qs,
+                           q_norm, k_norm, kc, vc, page_table, pos_ptr, 0, 0, part, H, HKV, block,
                            scale, n_rot, base, eps, rtab, rope_n);
         GD_LAUNCHED(ctx, "k_attn_decode");
         hipLaunchKernelGGL((k_attn_combine<256, uint16_t>), dim3(H), dim3(256), 0, ctx->stream,
@@ -1053,13 +1099,35 @@ extern "C" int gd_attn_paged(gd_ctx *ctx, const float *q, const uint16_t *k_cach
     int rc = check_attn(ctx, "gd_attn_paged", hd, n_head, n_head_kv, kv_dim, page_size, gated, gate);
     if (rc) return rc;
     GD_REQUIRE(ctx, T > 0 && lo >= 0 && lo < T, "gd_attn_paged: keys [lo=%d, T=%d) empty", lo, T);
-    // Key splits: a block of 32 keys for every wave, up to two workgroups per
+    // Few keys: a wave a key and q head.  Where a wave of k_attn_paged has one
+    // block (its q's operand, score tiles and merge are then most of its time)
+    // that is as fast or faster.  Call times, 24 / 4 heads x 256: 256, 732 and
+    // 1026 keys 8.4, 9.3 and 10.3 us (k_attn_paged 11.3, 11.7 and 10.8), 1536
+    // 14.1 (12.0), 4096 25.8 (13.0); 40 / 8 x 128: 256 keys 7.5 (8.2), 732 9.7
+    // (8.4), 1536 14.0 (9.8), 4096 28.4 (10.8); 16 / 8 x 128: 256 keys 7.7 (8.0),
+    // 732 8.0 (8.3), 1536 9.7 (9.1), 4096 18.5 (9.9).
+    if (2 * (int64_t)(T - lo) <= 9 * hd) {
+        const dim3 grid((unsigned)n_head, DSPLIT);
+        uint16_t *kc = const_cast<uint16_t *>(k_cache), *vc = const_cast<uint16_t *>(v_cache);
+#define GD_DECODE(HD_) \
+        hipLaunchKernelGGL((k_attn_decode<HD_, false>), grid, dim3(2 * HD_), 0, ctx->stream, q, HD_, nullptr, \
+                           nullptr, kc, vc, page_table, nullptr, T, lo, part, n_head, n_head_kv, page_size, \
+                           scale, 0, 0.f, 0.f, nullptr, 0); \
+        GD_LAUNCHED(ctx, "gd_attn_paged"); \
+        hipLaunchKernelGGL((k_attn_combine<HD_, float>), dim3(n_head), dim3(HD_), 0, ctx->stream, part, gate, \
+                           HD_, gated, out)
+        if (hd == 128) { GD_DECODE(128); } else { GD_DECODE(256); }
+#undef GD_DECODE
+        GD_LAUNCHED(ctx, "gd_attn_paged combine");
+        return GD_OK;
+    }
+    // Key splits: a block of 32 keys for every workgroup, up to two of them per
     // CU and what the combine weighs in one wave (64).  More than the 16 a
     // head that the caller's scratch holds go to the context's own scratch.
     const int G = n_head / n_head_kv, groups = n_head_kv * ((G + 7) / 8);
     const int cus = ctx->num_cus > 0 ? ctx->num_cus : 256;
     const int blocks = (T - lo + 31) / 32;
-    int ns = std::max(1, std::min({(blocks + PW - 1) / PW, MAX_SPLITS, std::max(DSPLIT, 2 * cus / groups)}));
+    int ns = std::max(1, std::min({blocks, MAX_SPLITS, std::max(DSPLIT, 2 * cus / groups)}));
     if (ns > DSPLIT &&
         (!ctx->attn_scratch || (size_t)n_head * ns * (hd + 2) * sizeof(float) > GD_ATTN_SCRATCH_BYTES))
         ns = DSPLIT;

@@ -143,12 +143,14 @@ def test_decode_and_batch_attention(ctx, hd, nh, nkv, page, T):
 
 @pytest.mark.parametrize("hd,nh,nkv,page,T,lo", [
     (128, 40, 8, 16, 1, 0), (256, 24, 4, 16, 33, 0), (128, 2, 2, 5, 31, 30), (256, 9, 1, 16, 64, 1),
+    (128, 16, 8, 16, 576, 0), (128, 40, 8, 16, 577, 0), (256, 9, 1, 16, 1155, 1), (128, 5, 1, 3, 2047, 0),
     (128, 34, 2, 16, 4099, 0), (256, 6, 1, 7, 4097, 100), (128, 16, 8, 16, 9000, 4999)])
 def test_decode_attention_key_blocks(ctx, hd, nh, nkv, page, T, lo):
     """One query over cached keys lo .. T-1 around the edges of the key blocks
-    and splits (one key, one past a block, several rounds of a wave), with one,
-    two, six and more than eight q heads a kv head: against f64 over the same
-    f16 cache within 3e-6 (22-bit q and weights, f32 sums)."""
+    and splits (one key, one past a block, several rounds of a wave) and of the
+    few keys (9/2 head dims) that go a wave a key, with one, two, five, six
+    and more than eight q heads a kv head: against f64 over the same f16 cache
+    within 3e-6 (22-bit q and weights, f32 sums)."""
     rng = np.random.default_rng(T + nh)
     kv_dim, npages = hd * nkv, (T + page - 1) // page + 1
     table = rng.permutation(npages).astype(np.int32)
