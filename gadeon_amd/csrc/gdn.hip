@@ -260,7 +260,49 @@ extern "C" int gd_rmsnorm_rows(gd_ctx *ctx, float *x, int d, int64_t rows, const
     return GD_OK;
 }
 
-// One 256-thread block per row of length n (the hidden size).
+constexpr int RMS_VEC = 4;       // pieces a thread: rows up to 8192
+// The row held in registers: a row is read once, 16 bytes a lane, with its
+// weights requested beside it.  Bound by two latencies of memory and the block's
+// sum; one float a lane in a loop, read twice, took 11.6 us for 27 as for 333
+// rows of 5120, this 2.5 and 4.5.
+template <int YT>
+__global__ __launch_bounds__(512) void gd_rmsnorm_vec_kernel(const float *x, const float *w, void *y, int n,
+                                                             float eps) {
+    __shared__ float red[8];
+    const int64_t row = blockIdx.x;
+    const float *xr = x + row * n;
+    f32x4 v[RMS_VEC], ww[RMS_VEC];
+    float ss = 0.0f;
+#pragma unroll
+    for (int k = 0; k < RMS_VEC; k++) {
+        const int i = 4 * (threadIdx.x + 512 * k);
+        if (i >= n) break;
+        v[k] = *(const f32x4 *)(xr + i);
+        ww[k] = *(const f32x4 *)(w + i);
+    }
+#pragma unroll
+    for (int k = 0; k < RMS_VEC; k++) {
+        if (4 * ((int)threadIdx.x + 512 * k) >= n) break;
+        ss += (v[k][0] * v[k][0] + v[k][1] * v[k][1]) + (v[k][2] * v[k][2] + v[k][3] * v[k][3]);
+    }
+    ss = gd_block_sum(ss, red);
+    const float s = 1.0f / sqrtf(ss / (float)n + eps);
+#pragma unroll
+    for (int k = 0; k < RMS_VEC; k++) {
+        const int i = 4 * (threadIdx.x + 512 * k);
+        if (i >= n) break;
+        const f32x4 o = v[k] * s * ww[k];
+        if (YT == GD_F32) {
+            *(f32x4 *)((float *)y + row * n + i) = o;
+        } else {
+            const uint32_t lo = (uint32_t)gd_f2h(o[0]) | ((uint32_t)gd_f2h(o[1]) << 16);
+            const uint32_t hi = (uint32_t)gd_f2h(o[2]) | ((uint32_t)gd_f2h(o[3]) << 16);
+            *(u32x2 *)((uint16_t *)y + row * n + i) = u32x2{lo, hi};
+        }
+    }
+}
+
+// One 256-thread block per row of length n, any n and alignment.
 template <int YT>
 __global__ void gd_rmsnorm_kernel(const float *x, const float *w, void *y, int64_t n, float eps) {
     __shared__ float red[4];
@@ -284,7 +326,17 @@ extern "C" int gd_rmsnorm(gd_ctx *ctx, const float *x, const float *w, void *y, 
     GD_REQUIRE(ctx, y_dtype == GD_F32 || y_dtype == GD_F16, "gd_rmsnorm: bad dtype");
     GD_REQUIRE(ctx, rows < (1LL << 31), "gd_rmsnorm: too many rows");
     if (!rows) return GD_OK;
-    if (y_dtype == GD_F32)
+    // Rows of whole 16-byte pieces that fit the registers (27 rows of 5120: 2.5
+    // us, a float a lane 11.6).
+    const bool vec = n % 4 == 0 && n <= 4 * 512 * RMS_VEC && (((uintptr_t)x | (uintptr_t)w) & 15) == 0 &&
+                     ((uintptr_t)y & (y_dtype == GD_F32 ? 15 : 7)) == 0;
+    if (vec && y_dtype == GD_F32)
+        hipLaunchKernelGGL(gd_rmsnorm_vec_kernel<GD_F32>, dim3((unsigned)rows), dim3(512), 0, ctx->stream, x, w,
+                           y, (int)n, eps);
+    else if (vec)
+        hipLaunchKernelGGL(gd_rmsnorm_vec_kernel<GD_F16>, dim3((unsigned)rows), dim3(512), 0, ctx->stream, x, w,
+                           y, (int)n, eps);
+    else if (y_dtype == GD_F32)
         hipLaunchKernelGGL(gd_rmsnorm_kernel<GD_F32>, dim3((unsigned)rows), dim3(256), 0,
                            ctx->stream, x, w, y, n, eps);
     else

@@ -110,6 +110,28 @@ def test_norms_and_elementwise(ctx):
         assert rel_diff(ctx.get(da, a.size, np.float32), ref) < 1e-5
 
 
+@pytest.mark.parametrize("n,rows,off", [(4, 3, 0), (2044, 5, 0), (2052, 2, 0), (8192, 3, 0), (8196, 2, 0),
+                                        (1026, 3, 0), (5120, 2, 1)])
+def test_rmsnorm_shapes(ctx, n, rows, off):
+    """Rows at the edges of a thread's 16-byte pieces, the longest held in
+    registers and one piece past it, a length and a start (off floats) that
+    are not whole pieces, in place as well: against f64, each element within
+    8 roundings of f32, half an ulp more in f16."""
+    x = np.concatenate([np.zeros(off, np.float32), O.lcg_normal(rows * n, 31)])
+    w = O.lcg_uniform(n, 32, 0.5, 1.5)
+    x64 = x[off:].reshape(rows, n).astype(np.float64)
+    want = x64 / np.sqrt((x64 ** 2).mean(1, keepdims=True) + EPS) * w
+    dx, dw, dy = ctx.put(x), ctx.put(w), ctx.alloc(x.nbytes)
+    tol = (8 + n ** 0.5 / 64) * 2.0 ** -24 * np.abs(want)
+    ctx.gd_rmsnorm(dx + 4 * off, dw, dy, ga.F16, n, rows, EPS)
+    got = ctx.get(dy, (rows, n), np.float16)
+    assert np.all(np.abs(got - want) <= tol + 2.0 ** -11 * np.abs(want) + 2.0 ** -25)
+    ctx.gd_rmsnorm(dx + 4 * off, dw, dx + 4 * off, ga.F32, n, rows, EPS)
+    assert np.all(np.abs(ctx.get(dx, x.size, np.float32)[off:].reshape(rows, n) - want) <= tol)
+    for p in (dx, dw, dy):
+        ctx.free(p)
+
+
 # ------------------------------------------------------------------ scan
 
 @pytest.mark.parametrize("nV,nK,dS", [(16, 16, 128), (16, 4, 128), (6, 3, 64)])
