@@ -186,6 +186,16 @@ struct AttnQ {
     float base, eps;
 };
 
+// Key splits of a prefill: split z of nz takes keys z ck .. (z+1) ck - 1 (ck a
+// multiple of 64) and leaves its unnormalized sums, [z][N][H][HD], and (max, sum
+// of weights) pairs, [z][N][H], for k_attn_prefill_combine; a query block whose
+// keys end before its split is done by the splits before it.
+struct AttnSplit {
+    float *acc;
+    float2 *ml;
+    int nz, ck;
+};
+
 // Causal prefill attention with the sigmoid output gate (Attention.swift:
 // 108-134), flash style on the matrix cores.  Block (head h, 64 queries):
 // wave w owns queries 16w .. 16w+15; keys stream through LDS in blocks of
@@ -201,10 +211,11 @@ struct AttnQ {
 // raw projection rows (qsrc.norm set) each lane group of a query holds all
 // of its dims (lane g: 32 ks + 8 g + e), so the q RMS norm is a sum over
 // the four groups and the rotation pairs (i, i + n_rot/2) lie in one lane
-// when n_rot/2 is a multiple of 32 (the host checks).
-template <int HD, typename OT>
+// when n_rot/2 is a multiple of 32 (the host checks).  SPLIT: a third grid
+// dimension of key splits (above).
+template <int HD, typename OT, bool SPLIT>
 __global__ __launch_bounds__(256) void k_attn_prefill(
-        AttnQ qsrc, const uint16_t *kc, const uint16_t *vc,
+        AttnQ qsrc, AttnSplit split, const uint16_t *kc, const uint16_t *vc,
         const int32_t *page_table, const int32_t *pos_ptr, int pos_add, OT *out, int H, int HKV,
         int N, int block, float scale, int gated) {
     constexpr int AK = prefill_keys<HD>();
@@ -226,7 +237,10 @@ __global__ __launch_bounds__(256) void k_attn_prefill(
     const int n = q0 + 16 * w + lq;                       // this lane's query
     const bool valid = n < N;
     const int my_pos = pos0 + (valid ? n : N - 1);
-    const int last = pos0 + min(q0 + AQ, N) - 1;          // last key any query here needs
+    // First key of the split and last key any query here needs of it.
+    const int kbeg = SPLIT ? (int)blockIdx.z * split.ck : 0;
+    const int last = SPLIT ? min(pos0 + min(q0 + AQ, N), kbeg + split.ck) - 1 : pos0 + min(q0 + AQ, N) - 1;
+    if (SPLIT && kbeg > last) return;
     // Staging: thread t loads dims d0 .. d0 + DPT - 1 of key t / TPK of the
     // block.  The loads run ahead of the arithmetic: block k0 + AK's K and V
     // rows are requested before block k0's MFMAs, and the page-table entry
@@ -244,8 +258,8 @@ __global__ __launch_bounds__(256) void k_attn_prefill(
             kv[CH + c] = *(const u32x4 *)(vc + base + 8 * c);
         }
     };
-    fetch(0, page_of(0));
-    int page_next = page_of(AK);
+    fetch(kbeg, page_of(kbeg));
+    int page_next = page_of(kbeg + AK);
     // q after the first key block's loads, so their latencies overlap.
     // B operand of S^T: q[n][32 ks + 8 g + e] * scale, split hi + lo.
     const int64_t qoff = (int64_t)(valid ? n : N - 1) * qsrc.tstride + (int64_t)h * qsrc.hstride;
@@ -306,7 +320,7 @@ __global__ __launch_bounds__(256) void k_attn_prefill(
 #pragma unroll
     for (int dt = 0; dt < HD / 16; dt++) acc[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
     float m = -INFINITY, l = 0.f;                         // this lane's keys only
-    for (int k0 = 0; k0 <= last; k0 += AK) {
+    for (int k0 = kbeg; k0 <= last; k0 += AK) {
         __syncthreads();
 #pragma unroll
         for (int c = 0; c < CH; c++) {
@@ -345,7 +359,10 @@ __global__ __launch_bounds__(256) void k_attn_prefill(
             }
         bmax = fmaxf(bmax, __shfl_xor(bmax, 16, 64));
         bmax = fmaxf(bmax, __shfl_xor(bmax, 32, 64));
-        const float mn = fmaxf(m, bmax);                  // finite: key k0 <= my_pos
+        // Finite: key k0 <= my_pos, unless the whole split lies behind the query
+        // (all weights 0).
+        float mn = fmaxf(m, bmax);
+        if (SPLIT && mn == -INFINITY) mn = -__FLT_MAX__;
         // The softmax exponents are <= 0 (or -inf for masked keys: 0), where
         // the hardware exp2 behind __expf is accurate to a few ulp.
         const float alpha = __expf(m - mn);
@@ -389,6 +406,14 @@ __global__ __launch_bounds__(256) void k_attn_prefill(
     // Total weight of query lq: the four lane groups' partial sums.
     l += __shfl_xor(l, 16, 64);
     l += __shfl_xor(l, 32, 64);
+    if (SPLIT) {
+        if (!valid) return;
+        const int64_t row = ((int64_t)blockIdx.z * N + n) * H + h;
+#pragma unroll
+        for (int dt = 0; dt < HD / 16; dt++) *(f32x4 *)(split.acc + row * HD + 16 * dt + 4 * g) = acc[dt];
+        if (g == 0) split.ml[row] = make_float2(m, l);
+        return;
+    }
     if (valid) {
         const float inv = 1.0f / l;
         const float *grow = qsrc.gate + (int64_t)n * qsrc.tstride + (int64_t)h * qsrc.hstride;
@@ -413,6 +438,38 @@ __global__ __launch_bounds__(256) void k_attn_prefill(
             }
         }
     }
+}
+
+// Sums the key splits of every (query, head) row, HD / 4 threads a row, four
+// dims each: split z takes part where n's query block reaches its keys.
+template <int HD>
+__global__ __launch_bounds__(256) void k_attn_prefill_combine(const float *gate, AttnSplit split, int pos0,
+                                                              float *out, int H, int N, int gated) {
+    constexpr int TPR = HD / 4;
+    const int64_t i = (int64_t)blockIdx.x * (256 / TPR) + threadIdx.x / TPR;   // row n H + h
+    if (i >= (int64_t)N * H) return;
+    const int n = (int)(i / H), d = 4 * (threadIdx.x % TPR);
+    const int keys = pos0 + min((n / AQ + 1) * AQ, N);    // keys of n's query block
+    const int nz = min(split.nz, (keys + split.ck - 1) / split.ck);
+    const int64_t zs = (int64_t)N * H;
+    float M = -INFINITY;
+    for (int z = 0; z < nz; z++) M = fmaxf(M, split.ml[z * zs + i].x);
+    float L = 0.f;
+    f32x4 a = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 4
+    for (int z = 0; z < nz; z++) {
+        const float2 ml = split.ml[z * zs + i];
+        const float f = __expf(ml.x - M);                 // split 0 holds key 0: M is a score
+        L += ml.y * f;
+        a += *(const f32x4 *)(split.acc + (z * zs + i) * HD + d) * f;
+    }
+    f32x4 r = a * (1.0f / L);
+    if (gated) {
+        const f32x4 gv = *(const f32x4 *)(gate + i * HD + d);
+#pragma unroll
+        for (int v = 0; v < 4; v++) r[v] *= gd_sigmoid(gv[v]);
+    }
+    *(f32x4 *)(out + i * HD + d) = r;
 }
 
 // ---------------------------------------------------------------- decode
@@ -643,6 +700,7 @@ __global__ __launch_bounds__(2 * HD) void k_attn_decode(
 // 2.2e-7, 3.2e-7.  With unscaled q and weights the low halves fell below
 // f16's normal range (3.4e-7).
 constexpr int PW = 4;           // waves
+constexpr int SPLIT_KEYS = 64, MAX_KEY_SPLITS = 32;   // fewest keys of a prefill's split, most splits
 constexpr float LOG2E = 1.4426950408889634f;
 template <int HD>
 __global__ __launch_bounds__(64 * PW) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_attn_paged(
@@ -977,8 +1035,8 @@ int gd_attn_prefill_launch(gd_ctx *ctx, int hd, const float *q, const float *gat
     const AttnQ qsrc{q, gate, q_tstride, q_hstride, q_norm, (const float2 *)rope_tab, rope_n, n_rot,
                      base, eps};
     const dim3 grid((unsigned)H, gd_blocks(N, AQ));
-#define GD_AP(HD_, OT_) hipLaunchKernelGGL((k_attn_prefill<HD_, OT_>), grid, dim3(256), 0, \
-        ctx->stream, qsrc, kc, vc, page_table, pos_ptr, pos_add, (OT_ *)out, H, HKV, N, block, \
+#define GD_AP(HD_, OT_) hipLaunchKernelGGL((k_attn_prefill<HD_, OT_, false>), grid, dim3(256), 0, \
+        ctx->stream, qsrc, AttnSplit{}, kc, vc, page_table, pos_ptr, pos_add, (OT_ *)out, H, HKV, N, block, \
         scale, gated)
     if (hd == 128) { if (out_dtype == GD_F16) GD_AP(128, uint16_t); else GD_AP(128, float); }
     else { if (out_dtype == GD_F16) GD_AP(256, uint16_t); else GD_AP(256, float); }
@@ -1158,6 +1216,38 @@ extern "C" int gd_attn_batch(gd_ctx *ctx, const float *q, const uint16_t *k_cach
     GD_REQUIRE(ctx, ((uintptr_t)q | (uintptr_t)out | (uintptr_t)(gated ? gate : q)) % 16 == 0,
                "gd_attn_batch: q, gate and out must be 16-byte aligned");
     if (!N) return GD_OK;
+    // Few queries over many keys leave most of the chip idle, each block a
+    // serial chain over all keys, 2.2 us per 32 of them at head dim 256: the
+    // keys are split, for up to two blocks a CU and what the context's scratch
+    // holds, from 64 keys a split (about what the partials' round trip and the
+    // combine cost).  24 / 4 x 256, 16 queries after 112 keys 22.4 -> 15.7 us,
+    // 500 50.3 -> 21.6, 4000 288 -> 51; 100 after 4000 295 -> 109; 200 after
+    // none 29.7, unsplit (the chip is filled from 11 query blocks on).
+    //   Head dim 128 stays unsplit: its kernel rounds the high half of some q
+    // from the fused product and the low half from the rounded one, which ones
+    // depends on the compiled variant, and outputs would differ between a split
+    // and an unsplit call by up to 7e-4 of their size.
+    const int64_t keys = (int64_t)base_pos + N;
+    const int64_t units = (int64_t)n_head * gd_blocks(N, AQ), row = (int64_t)N * n_head * (hd * 4 + 8);
+    const int cus = ctx->num_cus > 0 ? ctx->num_cus : 256;
+    int64_t nz = hd != 256 ? 0 : std::min({(int64_t)MAX_KEY_SPLITS, 2 * (int64_t)cus / units, keys / SPLIT_KEYS,
+                           ctx->attn_scratch ? (int64_t)GD_ATTN_SCRATCH_BYTES / row : 0});
+    if (nz > 1) {
+        const int64_t ck = ((keys + nz - 1) / nz + 63) / 64 * 64;
+        nz = (keys + ck - 1) / ck;
+        const AttnQ qsrc{q, gated ? gate : q, (int64_t)n_head * hd, hd, nullptr, nullptr, 0, 0, 0.f, 0.f};
+        const AttnSplit split{ctx->attn_scratch, (float2 *)(ctx->attn_scratch + nz * N * n_head * hd), (int)nz,
+                              (int)ck};
+        const dim3 grid((unsigned)n_head, gd_blocks(N, AQ), (unsigned)nz);
+        hipLaunchKernelGGL((k_attn_prefill<256, float, true>), grid, dim3(256), 0, ctx->stream, qsrc, split,
+                           k_cache, v_cache, page_table, nullptr, base_pos, out, n_head, n_head_kv, (int)N,
+                           page_size, scale, gated);
+        GD_LAUNCHED(ctx, "k_attn_prefill");
+        hipLaunchKernelGGL(k_attn_prefill_combine<256>, dim3(gd_blocks(N * n_head, 4)), dim3(256), 0,
+                           ctx->stream, gate, split, base_pos, out, n_head, (int)N, gated);
+        GD_LAUNCHED(ctx, "k_attn_prefill_combine");
+        return GD_OK;
+    }
     return gd_attn_prefill_launch(ctx, hd, q, gated ? gate : q, (int64_t)n_head * hd, hd, nullptr, 0,
                                   0.f, 0.f, nullptr, 0, k_cache, v_cache, page_table, nullptr,
                                   base_pos, out, GD_F32, n_head, n_head_kv, (int)N, page_size,

@@ -166,6 +166,33 @@ def test_decode_attention_key_blocks(ctx, hd, nh, nkv, page, T, lo):
         ctx.free(p)
 
 
+@pytest.mark.parametrize("hd,nh,nkv,page,N,base", [
+    (256, 6, 2, 16, 1, 127), (256, 8, 2, 5, 3, 700), (256, 4, 4, 16, 65, 1000), (256, 4, 1, 16, 200, 0),
+    (256, 2, 1, 7, 64, 4100)])
+def test_prefill_attention_key_splits(ctx, hd, nh, nkv, page, N, base):
+    """Few queries over many cached keys (head dim 256): two splits and the most,
+    query blocks that end before the last splits, queries that precede a whole
+    split of their block, rows short of a block: against f64 over the same f16
+    cache (q and weights split into 22 bits, f32 sums: 1e-5 of the output)."""
+    rng = np.random.default_rng(N + base)
+    T, kv_dim = N + base, hd * nkv
+    npages = (T + page - 1) // page + 1
+    table = rng.permutation(npages).astype(np.int32)
+    K, V = (rng.standard_normal((npages, page, nkv, hd)).astype(np.float16) for _ in range(2))
+    q, gate = (rng.standard_normal((N, nh, hd)).astype(np.float32) for _ in range(2))
+    bufs = [ctx.put(a) for a in (q, K.view(np.uint16), V.view(np.uint16), table, gate)]
+    out = ctx.alloc(q.nbytes)
+    ctx.gd_attn_batch(*bufs, out, hd, nh, nkv, kv_dim, page, C.c_float(1 / np.sqrt(hd)), base, N, 1, 0)
+    got = ctx.get(out, q.shape, np.float32)
+    rows = lambda a: a[table].reshape(npages * page, nkv, hd)
+    Kr, Vr = rows(K), rows(V)
+    for n in range(N):
+        want = ref_attention(q[n], Kr[:base + n + 1], Vr[:base + n + 1], gate[n], nkv, base + n + 1)
+        assert rel_diff(got[n], want) < 1e-5, n
+    for p in (*bufs, out):
+        ctx.free(p)
+
+
 def test_attention_rejects_bad_shapes(ctx):
     d = ctx.alloc(64)
     lib = ctx.lib
