@@ -249,13 +249,44 @@ __global__ void gd_rmsnorm_rows_kernel(float *x, int d, int64_t rows, const floa
     for (int i = lane; i < d; i += 64) r[i] = r[i] * s * w[i];
 }
 
+// Rows of 4 L elements, a row in L lanes' registers (16 bytes a lane) and four
+// rows a thread in flight.  Bound by HBM: 48000 rows of 128 (49 MB) 8.7 us,
+// one row a wave and 4 bytes a lane 14.0.
+template <int L>
+__global__ __launch_bounds__(256) void gd_rmsnorm_rows_vec_kernel(float *x, int64_t rows, const float *w, float eps) {
+    constexpr int NR = 4, D = 4 * L, G = 256 / L;
+    const int l = threadIdx.x % L;
+    const int64_t r0 = (int64_t)blockIdx.x * (G * NR) + threadIdx.x / L;
+    const f32x4 wv = *(const f32x4 *)(w + 4 * l);
+    f32x4 v[NR];
+#pragma unroll
+    for (int k = 0; k < NR; k++) v[k] = *(const f32x4 *)(x + min(r0 + G * k, rows - 1) * D + 4 * l);
+#pragma unroll
+    for (int k = 0; k < NR; k++) {
+        float ss = (v[k][0] * v[k][0] + v[k][1] * v[k][1]) + (v[k][2] * v[k][2] + v[k][3] * v[k][3]);
+#pragma unroll
+        for (int o = L / 2; o >= 1; o >>= 1) ss += __shfl_xor(ss, o, 64);
+        const float s = 1.0f / sqrtf(ss / (float)D + eps);
+        if (r0 + G * k < rows) *(f32x4 *)(x + (r0 + G * k) * D + 4 * l) = v[k] * s * wv;
+    }
+}
+
 extern "C" int gd_rmsnorm_rows(gd_ctx *ctx, float *x, int d, int64_t rows, const float *w,
                                float eps) {
     GD_CHECK_CTX(ctx);
     GD_REQUIRE(ctx, x && w && d > 0 && rows >= 0, "gd_rmsnorm_rows: bad arguments");
     if (!rows) return GD_OK;
-    hipLaunchKernelGGL(gd_rmsnorm_rows_kernel, dim3(gd_blocks(rows, 4)), dim3(256), 0,
-                       ctx->stream, x, d, rows, w, eps);
+    // The head dims of the models (14.0 -> 8.7 us, 48000 rows of 128; 16-byte rows).
+    const bool al = (((uintptr_t)x | (uintptr_t)w) & 15) == 0;
+    if (d == 128 && al)
+        hipLaunchKernelGGL(gd_rmsnorm_rows_vec_kernel<32>, dim3(gd_blocks(rows, 32)), dim3(256), 0, ctx->stream, x,
+                           rows, w, eps);
+    else if (d == 256 && al)
+        hipLaunchKernelGGL(gd_rmsnorm_rows_vec_kernel<64>, dim3(gd_blocks(rows, 16)), dim3(256), 0, ctx->stream, x,
+                           rows, w, eps);
+    else
+        hipLaunchKernelGGL(gd_rmsnorm_rows_kernel, dim3(gd_blocks(rows, 4)), dim3(256), 0,
+                           ctx->stream, x, d, rows, w, eps);
     GD_LAUNCHED(ctx, "rmsnorm_rows");
     return GD_OK;
 }

@@ -132,6 +132,25 @@ def test_rmsnorm_shapes(ctx, n, rows, off):
         ctx.free(p)
 
 
+@pytest.mark.parametrize("d,rows,off", [(128, 1, 0), (128, 33, 0), (128, 63, 1), (256, 17, 0), (256, 5, 2),
+                                        (64, 9, 0)])
+def test_rmsnorm_rows_shapes(ctx, d, rows, off):
+    """Head dims 128 and 256 short of a block's rows, unaligned starts and
+    another head dim: against f64 within 8 roundings of f32, rows past the
+    last untouched."""
+    x = O.lcg_normal(off + (rows + 1) * d, 33)
+    w = O.lcg_uniform(d, 34, 0.5, 1.5)
+    x64 = x[off:off + rows * d].reshape(rows, d).astype(np.float64)
+    want = x64 / np.sqrt((x64 ** 2).mean(1, keepdims=True) + EPS) * w
+    dx, dw = ctx.put(x), ctx.put(w)
+    ctx.gd_rmsnorm_rows(dx + 4 * off, d, rows, dw, EPS)
+    got = ctx.get(dx, x.size, np.float32)
+    assert np.all(np.abs(got[off:off + rows * d].reshape(rows, d) - want) <= 10 * 2.0 ** -24 * np.abs(want))
+    assert np.array_equal(got[:off], x[:off]) and np.array_equal(got[off + rows * d:], x[off + rows * d:])
+    for p in (dx, dw):
+        ctx.free(p)
+
+
 # ------------------------------------------------------------------ scan
 
 @pytest.mark.parametrize("nV,nK,dS", [(16, 16, 128), (16, 4, 128), (6, 3, 64)])
