@@ -92,7 +92,8 @@ template <int V> __device__ __forceinline__ void st_floats(float *p, const Float
 // channels 327 us with one thread per channel walking all tokens (40
 // workgroups, one load in flight each), 20 us here (4.1 TB/s of x and out; a
 // large copy runs at 4.7).  Only tile 0 reads the ring
-// (TT >= KC - 1), so it alone advances it, after its reads.
+// (TT >= KC - 1), so it alone advances it, after its reads, to the last KC - 1
+// inputs (N >= KC - 1: fewer tokens take the serial kernel).
 template <int KC, int V, int TT>
 __global__ __launch_bounds__(256) void gd_conv_tile_kernel(const float *__restrict__ x, float *ring,
                                                            const float *__restrict__ cw,
@@ -102,7 +103,7 @@ __global__ __launch_bounds__(256) void gd_conv_tile_kernel(const float *__restri
     const int c = (blockIdx.x * 256 + threadIdx.x) * V;
     if (c >= convDim) return;
     const int64_t n0 = (int64_t)blockIdx.y * TT;
-    Floats<V> win[TT + KC - 1], old[KC];                 // win[j]: token n0 - (KC - 1) + j
+    Floats<V> win[TT + KC - 1];                          // win[j]: token n0 - (KC - 1) + j
     float w[V][KC];
 #pragma unroll
     for (int j = 0; j < TT + KC - 1; j++) {
@@ -115,10 +116,7 @@ __global__ __launch_bounds__(256) void gd_conv_tile_kernel(const float *__restri
         for (int j = 0; j < KC; j++) w[i][j] = cw[(int64_t)(c + i) * KC + j];
     if (n0 == 0) {
 #pragma unroll
-        for (int j = 0; j + 1 < KC; j++) {
-            old[j] = ld_floats<V>(ring + (int64_t)j * convDim + c);
-            win[j] = old[j];
-        }
+        for (int j = 0; j + 1 < KC; j++) win[j] = ld_floats<V>(ring + (int64_t)j * convDim + c);
     }
 #pragma unroll
     for (int t = 0; t < TT; t++) {
@@ -134,22 +132,9 @@ __global__ __launch_bounds__(256) void gd_conv_tile_kernel(const float *__restri
         st_floats<V>(out + (n0 + t) * convDim + c, y);
     }
     if (n0 == 0) {
-        // The inputs of tokens N - KC + 1 .. N - 1 (the old ring's where those
-        // precede token 0: row KC - 1 + m).
 #pragma unroll
-        for (int j = 0; j + 1 < KC; j++) {
-            const int64_t m = N - (KC - 1) + j;
-            Floats<V> r;
-            if (m >= 0) {
-                r = ld_floats<V>(x + m * convDim + c);
-            } else {
-                r = old[0];
-#pragma unroll
-                for (int k = 1; k + 1 < KC; k++)
-                    if (KC - 1 + m == k) r = old[k];
-            }
-            st_floats<V>(ring + (int64_t)j * convDim + c, r);
-        }
+        for (int j = 0; j + 1 < KC; j++)
+            st_floats<V>(ring + (int64_t)j * convDim + c, ld_floats<V>(x + (N - (KC - 1) + j) * convDim + c));
     }
 }
 
@@ -158,9 +143,16 @@ __global__ __launch_bounds__(256) void gd_conv_tile_kernel(const float *__restri
 // where rows keep 16-byte alignment.  Tiles of 16 tokens (a fifth more rows
 // read than the input has) once they fill the chip twice over, else of 4 (8
 // where the window is longer), so that short inputs spread over more CUs.
+//   Up to 10 tokens walk the channels: 1.8 us and 0.2 a token for a chain of
+// calls, at 4096 to 10240 channels alike, where the tiles, a quarter of the
+// workgroups and a window of loads each, take 2.9 (one token) to 3.7 (from 4
+// on): 1, 4, 8 and 12 tokens 2.0, 2.4, 3.2 and 4.1 us (tiles 2.9, 3.7, 3.7, 3.7).
+constexpr int CONV_SERIAL = 10;
 template <int KC>
 static bool launch_conv_tiles(gd_ctx *ctx, const float *x, float *ring, const float *cw, float *out,
                               int convDim, int64_t N) {
+    static_assert(CONV_SERIAL >= KC - 1, "the tiles advance the ring from x alone");
+    if (N <= CONV_SERIAL) return false;
     auto apart = [](const void *a, size_t an, const void *b, size_t bn) {
         const uintptr_t p = (uintptr_t)a, q = (uintptr_t)b;
         return p + an <= q || q + bn <= p;

@@ -76,6 +76,15 @@ def test_conv_tiles(ctx, convDim, kc, N, off):
         assert np.array_equal(ctx.get(dr, ring_ref.size, np.float32), ring_ref)
 
 
+@pytest.mark.parametrize("convDim,kc,N,off", [
+    (260, 4, 10, 0), (260, 4, 11, 0), (257, 1, 11, 0), (512, 8, 11, 0), (516, 8, 10, 0), (512, 2, 12, 0),
+    (256, 8, 13, 1)])
+def test_conv_fewest_tiled_tokens(ctx, convDim, kc, N, off):
+    """The last token count that walks the channels and the first ones in
+    tiles, whose last inputs replace the whole ring: as test_conv_tiles."""
+    test_conv_tiles(ctx, convDim, kc, N, off)
+
+
 def test_norms_and_elementwise(ctx):
     N, nK, d, convDim = 9, 16, 128, 6144
     x = O.lcg_normal(N * convDim, 21).reshape(N, convDim)

@@ -1,0 +1,53 @@
+"""The rules that send a call to one of two kernels, by time: where an entry
+has a second kernel that a call can be put on (an output over its input, a
+start off 16-byte alignment, a forced plan), the one that the rule picks for
+the plain call is not the slower one.  Each side is a recorded chain of calls,
+the fastest of several replays; 1.25 leaves room for the placement of buffers
+and for the other kernel's own small costs, and the rules that these tests
+were written against were off by 1.3 to 3."""
+import ctypes as C
+
+import pytest
+
+import gadeon_amd as ga
+
+pytestmark = pytest.mark.gpu
+
+EPS = 1e-6
+SLACK = 1.25
+
+
+def chain_ms(ctx, call, n=50, replays=12):
+    """Fastest replay of n recorded calls, after one direct call (workspaces)."""
+    call()
+    ctx.gd_graph_begin()
+    for _ in range(n):
+        call()
+    g, ms, best = C.c_void_p(), C.c_float(), 1e9
+    ctx.gd_graph_end(C.byref(g))
+    for _ in range(replays):
+        ctx.gd_timer_start()
+        ctx.gd_graph_launch(g)
+        ctx.gd_timer_stop(C.byref(ms))
+        best = min(best, ms.value)
+    ctx.lib.gd_graph_destroy(g)
+    return best
+
+
+def zeros(ctx, nbytes):
+    p = ctx.alloc(nbytes)
+    ctx.gd_fill_u32(p, 0, nbytes // 4)
+    return p
+
+
+@pytest.mark.parametrize("N", [1, 4, 8, 10])
+def test_conv_few_tokens(ctx, N):
+    """Few tokens against the token-serial kernel, which a call takes whose
+    output replaces its input."""
+    cd = 8192
+    x, o, ring, cw = (zeros(ctx, n * cd * 4) for n in (N, N, 3, 4))
+    picked = chain_ms(ctx, lambda: ctx.gd_gdn_conv(x, ring, cw, o, cd, 4, N))
+    serial = chain_ms(ctx, lambda: ctx.gd_gdn_conv(x, ring, cw, x, cd, 4, N))
+    assert picked < SLACK * serial
+    for p in (x, o, ring, cw):
+        ctx.free(p)
