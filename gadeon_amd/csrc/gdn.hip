@@ -283,36 +283,35 @@ extern "C" int gd_rmsnorm_rows(gd_ctx *ctx, float *x, int d, int64_t rows, const
     return GD_OK;
 }
 
-constexpr int RMS_VEC = 4;       // pieces a thread: rows up to 8192
-// The row held in registers: a row is read once, 16 bytes a lane, with its
-// weights requested beside it.  Bound by two latencies of memory and the block's
-// sum; one float a lane in a loop, read twice, took 11.6 us for 27 as for 333
-// rows of 5120, this 2.5 and 4.5.
-template <int YT>
-__global__ __launch_bounds__(512) void gd_rmsnorm_vec_kernel(const float *x, const float *w, void *y, int n,
-                                                             float eps) {
-    __shared__ float red[8];
+// The row held in the registers of NT threads, NP 16-byte pieces each: a row is
+// read once, with its weights requested beside it.  Bound by two latencies of
+// memory and the block's sum; one float a lane in a loop, read twice, took 11.6
+// us for 27 as for 333 rows of 5120, this (512 x 4) 2.5 and 4.5.
+template <int YT, int NT, int NP>
+__global__ __launch_bounds__(NT) void gd_rmsnorm_vec_kernel(const float *x, const float *w, void *y, int n,
+                                                            float eps) {
+    __shared__ float red[NT / 64];
     const int64_t row = blockIdx.x;
     const float *xr = x + row * n;
-    f32x4 v[RMS_VEC], ww[RMS_VEC];
+    f32x4 v[NP], ww[NP];
     float ss = 0.0f;
 #pragma unroll
-    for (int k = 0; k < RMS_VEC; k++) {
-        const int i = 4 * (threadIdx.x + 512 * k);
+    for (int k = 0; k < NP; k++) {
+        const int i = 4 * (threadIdx.x + NT * k);
         if (i >= n) break;
         v[k] = *(const f32x4 *)(xr + i);
         ww[k] = *(const f32x4 *)(w + i);
     }
 #pragma unroll
-    for (int k = 0; k < RMS_VEC; k++) {
-        if (4 * ((int)threadIdx.x + 512 * k) >= n) break;
+    for (int k = 0; k < NP; k++) {
+        if (4 * ((int)threadIdx.x + NT * k) >= n) break;
         ss += (v[k][0] * v[k][0] + v[k][1] * v[k][1]) + (v[k][2] * v[k][2] + v[k][3] * v[k][3]);
     }
     ss = gd_block_sum(ss, red);
     const float s = 1.0f / sqrtf(ss / (float)n + eps);
 #pragma unroll
-    for (int k = 0; k < RMS_VEC; k++) {
-        const int i = 4 * (threadIdx.x + 512 * k);
+    for (int k = 0; k < NP; k++) {
+        const int i = 4 * (threadIdx.x + NT * k);
         if (i >= n) break;
         const f32x4 o = v[k] * s * ww[k];
         if (YT == GD_F32) {
@@ -350,21 +349,24 @@ extern "C" int gd_rmsnorm(gd_ctx *ctx, const float *x, const float *w, void *y, 
     GD_REQUIRE(ctx, rows < (1LL << 31), "gd_rmsnorm: too many rows");
     if (!rows) return GD_OK;
     // Rows of whole 16-byte pieces that fit the registers (27 rows of 5120: 2.5
-    // us, a float a lane 11.6).
-    const bool vec = n % 4 == 0 && n <= 4 * 512 * RMS_VEC && (((uintptr_t)x | (uintptr_t)w) & 15) == 0 &&
+    // us, a float a lane 11.6), in 512 threads, or in 128 where those hold the
+    // row.  A launch holds fewer than 2^32 threads: rows past that go a float a lane.
+    const int nt = n <= 512 ? 128 : 512;
+    const bool vec = n % 4 == 0 && n <= 8192 && (uint64_t)rows * nt < (1ULL << 32) &&
+                     (((uintptr_t)x | (uintptr_t)w) & 15) == 0 &&
                      ((uintptr_t)y & (y_dtype == GD_F32 ? 15 : 7)) == 0;
-    if (vec && y_dtype == GD_F32)
-        hipLaunchKernelGGL(gd_rmsnorm_vec_kernel<GD_F32>, dim3((unsigned)rows), dim3(512), 0, ctx->stream, x, w,
-                           y, (int)n, eps);
-    else if (vec)
-        hipLaunchKernelGGL(gd_rmsnorm_vec_kernel<GD_F16>, dim3((unsigned)rows), dim3(512), 0, ctx->stream, x, w,
-                           y, (int)n, eps);
-    else if (y_dtype == GD_F32)
-        hipLaunchKernelGGL(gd_rmsnorm_kernel<GD_F32>, dim3((unsigned)rows), dim3(256), 0,
-                           ctx->stream, x, w, y, n, eps);
-    else
-        hipLaunchKernelGGL(gd_rmsnorm_kernel<GD_F16>, dim3((unsigned)rows), dim3(256), 0,
-                           ctx->stream, x, w, y, n, eps);
+#define GD_RMS(K_, NT_, N_) hipLaunchKernelGGL(K_, dim3((unsigned)rows), dim3(NT_), 0, ctx->stream, x, w, y, N_, eps)
+    if (vec && nt == 128) {
+        if (y_dtype == GD_F32) GD_RMS((gd_rmsnorm_vec_kernel<GD_F32, 128, 1>), 128, (int)n);
+        else GD_RMS((gd_rmsnorm_vec_kernel<GD_F16, 128, 1>), 128, (int)n);
+    } else if (vec) {
+        if (y_dtype == GD_F32) GD_RMS((gd_rmsnorm_vec_kernel<GD_F32, 512, 4>), 512, (int)n);
+        else GD_RMS((gd_rmsnorm_vec_kernel<GD_F16, 512, 4>), 512, (int)n);
+    } else {
+        if (y_dtype == GD_F32) GD_RMS(gd_rmsnorm_kernel<GD_F32>, 256, n);
+        else GD_RMS(gd_rmsnorm_kernel<GD_F16>, 256, n);
+    }
+#undef GD_RMS
     GD_LAUNCHED(ctx, "rmsnorm");
     return GD_OK;
 }

@@ -141,6 +141,13 @@ def test_rmsnorm_shapes(ctx, n, rows, off):
         ctx.free(p)
 
 
+@pytest.mark.parametrize("n,rows,off", [(64, 7, 0), (508, 3, 0), (512, 2, 0), (516, 2, 0)])
+def test_rmsnorm_row_threads(ctx, n, rows, off):
+    """Rows short of, at and past the longest that 128 threads hold: as
+    test_rmsnorm_shapes."""
+    test_rmsnorm_shapes(ctx, n, rows, off)
+
+
 @pytest.mark.parametrize("d,rows,off", [(128, 1, 0), (128, 33, 0), (128, 63, 1), (256, 17, 0), (256, 5, 2),
                                         (64, 9, 0)])
 def test_rmsnorm_rows_shapes(ctx, d, rows, off):

@@ -7,6 +7,7 @@ and for the other kernel's own small costs, and the rules that these tests
 were written against were off by 1.3 to 3."""
 import ctypes as C
 
+import numpy as np
 import pytest
 
 import gadeon_amd as ga
@@ -50,4 +51,27 @@ def test_conv_few_tokens(ctx, N):
     serial = chain_ms(ctx, lambda: ctx.gd_gdn_conv(x, ring, cw, x, cd, 4, N))
     assert picked < SLACK * serial
     for p in (x, o, ring, cw):
+        ctx.free(p)
+
+
+@pytest.mark.parametrize("n,rows", [(64, 20000), (128, 4000), (512, 20000), (1024, 20000)])
+def test_rmsnorm_short_rows(ctx, n, rows):
+    """Many short rows against the kernel for any alignment (x one float off)."""
+    x, w, y = zeros(ctx, rows * n * 4 + 16), zeros(ctx, n * 4), zeros(ctx, rows * n * 4)
+    picked = chain_ms(ctx, lambda: ctx.gd_rmsnorm(x, w, y, ga.F32, n, rows, EPS), 20)
+    general = chain_ms(ctx, lambda: ctx.gd_rmsnorm(x + 4, w, y, ga.F32, n, rows, EPS), 20)
+    assert picked < SLACK * general
+    for p in (x, w, y):
+        ctx.free(p)
+
+
+def test_rmsnorm_many_rows(ctx):
+    """2^23 rows of 516: 512 threads a row are more than one launch holds."""
+    n, rows = 516, 1 << 23
+    x, w = ctx.alloc(rows * n * 4), ctx.put(np.ones(n, np.float32))
+    ctx.gd_fill_u32(x, int(np.float32(3).view(np.uint32)), rows * n)
+    ctx.gd_rmsnorm(x, w, x, ga.F32, n, rows, EPS)
+    for r in (0, rows // 2, rows - 1):
+        assert np.allclose(ctx.get(x + r * n * 4, n, np.float32), 1, rtol=1e-6)
+    for p in (x, w):
         ctx.free(p)
