@@ -1164,7 +1164,10 @@ extern "C" int gd_attn_paged(gd_ctx *ctx, const float *q, const uint16_t *k_cach
     // 14.1 (12.0), 4096 25.8 (13.0); 40 / 8 x 128: 256 keys 7.5 (8.2), 732 9.7
     // (8.4), 1536 14.0 (9.8), 4096 28.4 (10.8); 16 / 8 x 128: 256 keys 7.7 (8.0),
     // 732 8.0 (8.3), 1536 9.7 (9.1), 4096 18.5 (9.9).
-    if (2 * (int64_t)(T - lo) <= 9 * hd) {
+    // Inputs off 16-byte alignment, which k_attn_paged loads q, K and V by, take
+    // it at any length.
+    const bool aligned = ((uintptr_t)q | (uintptr_t)k_cache | (uintptr_t)v_cache) % 16 == 0;
+    if (!aligned || 2 * (int64_t)(T - lo) <= 9 * hd) {
         const dim3 grid((unsigned)n_head, DSPLIT);
         uint16_t *kc = const_cast<uint16_t *>(k_cache), *vc = const_cast<uint16_t *>(v_cache);
 #define GD_DECODE(HD_) \

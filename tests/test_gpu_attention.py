@@ -166,6 +166,37 @@ def test_decode_attention_key_blocks(ctx, hd, nh, nkv, page, T, lo):
         ctx.free(p)
 
 
+@pytest.mark.parametrize("hd,nh,nkv", [(128, 10, 2), (256, 6, 1)])
+@pytest.mark.parametrize("off", [(4, 0, 0), (0, 4, 0), (0, 0, 4), (8, 8, 8), (0, 0, 0)])
+def test_decode_attention_alignment(ctx, hd, nh, nkv, off):
+    """q, K or V short of 16-byte alignment (off, bytes), with more keys than
+    the few-keys rule takes: the kernel of 16-byte loads is not launched, and
+    either kernel's result is within 3e-6 of f64."""
+    page, T = 16, 3000
+    rng = np.random.default_rng(hd + sum(off))
+    kv_dim, npages = hd * nkv, T // page + 1
+    table = rng.permutation(npages).astype(np.int32)
+    K, V = (rng.standard_normal((npages, page, nkv, hd)).astype(np.float16) for _ in range(2))
+    q, gate = (rng.standard_normal((nh, hd)).astype(np.float32) for _ in range(2))
+    bufs = [ctx.alloc(a.nbytes + 16) for a in (q, K, V)]
+    at = [b + o for b, o in zip(bufs, off)]
+    for p, a in zip(at, (q, K.view(np.uint16), V.view(np.uint16))):
+        ctx.set(p, a)
+    dt, dg = ctx.put(table), ctx.put(gate)
+    out, part = ctx.alloc(nh * hd * 4), ctx.alloc(nh * 16 * (hd + 2) * 4)
+    ctx.gd_fill_u32(part, 0xffffffff, nh * 16 * (hd + 2))
+    ctx.gd_attn_paged(*at, dt, dg, out, part, hd, nh, nkv, T, kv_dim, page, C.c_float(1 / np.sqrt(hd)), 1, 0)
+    rows = lambda a: a[table].reshape(npages * page, nkv, hd)[:T]
+    want = ref_attention(q, rows(K), rows(V), gate, nkv, T)
+    assert rel_diff(ctx.get(out, (nh, hd), np.float32), want) < 3e-6
+    # 16-byte loads need aligned inputs: without them the call has to be the
+    # wave-a-key kernel's, whose 16 splits a head fill the caller's scratch.
+    used = np.isfinite(ctx.get(part, nh * 16 * (hd + 2), np.float32)).all()
+    assert used == any(off)
+    for p in (*bufs, dt, dg, out, part):
+        ctx.free(p)
+
+
 @pytest.mark.parametrize("hd,nh,nkv,page,N,base", [
     (256, 6, 2, 16, 1, 127), (256, 8, 2, 5, 3, 700), (256, 4, 4, 16, 65, 1000), (256, 4, 1, 16, 200, 0),
     (256, 2, 1, 7, 64, 4100)])
