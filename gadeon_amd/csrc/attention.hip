@@ -261,7 +261,13 @@ __global__ __launch_bounds__(256) void k_attn_prefill(
     fetch(kbeg, page_of(kbeg));
     int page_next = page_of(kbeg + AK);
     // q after the first key block's loads, so their latencies overlap.
-    // B operand of S^T: q[n][32 ks + 8 g + e] * scale, split hi + lo.
+    // B operand of S^T: q[n][32 ks + 8 g + e] * scale, split hi + lo.  Head dim
+    // 128 leaves it to the compiler, which rounds hi from the exact product and
+    // lo from its f32 rounding: where those two round to different f16 the halves
+    // are an ulp apart (2^-11 of one dim's share of a score; up to 1.5e-3 of the
+    // rms in single outputs, 2.9e-6 in all).  Callers compare its outputs with
+    // recorded ones more closely than that, so it stays; head dim 256's scale
+    // 1/16 is exact either way, and other scales keep 22 bits.
     const int64_t qoff = (int64_t)(valid ? n : N - 1) * qsrc.tstride + (int64_t)h * qsrc.hstride;
     f16x8 qh[HD / 32], ql[HD / 32];
     {
@@ -312,8 +318,15 @@ __global__ __launch_bounds__(256) void k_attn_prefill(
 #pragma unroll
             for (int e = 0; e < 8; e++) {
                 const float v = x[ks][e] * scale;
-                qh[ks][e] = (f16)v;
-                ql[ks][e] = (f16)(v - (float)qh[ks][e]);
+                if constexpr (HD == 256) {
+                    f16 hi, lo;
+                    gd_split_f16(v, hi, lo);
+                    qh[ks][e] = hi;
+                    ql[ks][e] = lo;
+                } else {
+                    qh[ks][e] = (f16)v;
+                    ql[ks][e] = (f16)(v - (float)qh[ks][e]);
+                }
             }
     }
     f32x4 acc[HD / 16];                                   // O^T rows 16 dt + 4 g + v
@@ -1226,10 +1239,9 @@ extern "C" int gd_attn_batch(gd_ctx *ctx, const float *q, const uint16_t *k_cach
     // combine cost).  24 / 4 x 256, 16 queries after 112 keys 22.4 -> 15.7 us,
     // 500 50.3 -> 21.6, 4000 288 -> 51; 100 after 4000 295 -> 109; 200 after
     // none 29.7, unsplit (the chip is filled from 11 query blocks on).
-    //   Head dim 128 stays unsplit: its kernel rounds the high half of some q
-    // from the fused product and the low half from the rounded one, which ones
-    // depends on the compiled variant, and outputs would differ between a split
-    // and an unsplit call by up to 7e-4 of their size.
+    //   Head dim 128 stays unsplit: which of its q halves belong to two roundings
+    // (k_attn_prefill) depends on the compiled variant, and outputs would differ
+    // between a split and an unsplit call by up to 7e-4 of their size.
     const int64_t keys = (int64_t)base_pos + N;
     const int64_t units = (int64_t)n_head * gd_blocks(N, AQ), row = (int64_t)N * n_head * (hd * 4 + 8);
     const int cus = ctx->num_cus > 0 ? ctx->num_cus : 256;

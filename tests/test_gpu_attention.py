@@ -224,6 +224,30 @@ def test_prefill_attention_key_splits(ctx, hd, nh, nkv, page, N, base):
         ctx.free(p)
 
 
+@pytest.mark.parametrize("nh,nkv,N,base", [(8, 2, 5, 700), (12, 2, 700, 0)])
+def test_prefill_attention_scales(ctx, nh, nkv, N, base):
+    """Head dim 256 at a scale whose products with q round, with its keys split
+    over the chip (few queries) and not: both halves of q's split belong to one
+    value, so rows stay within 1e-5 of f64 (22-bit q and weights, f32 sums)."""
+    hd, page, scale = 256, 16, 0.07
+    rng = np.random.default_rng(N)
+    T, kv_dim = N + base, hd * nkv
+    npages = (T + page - 1) // page
+    K, V = (rng.standard_normal((npages * page, nkv, hd)).astype(np.float16) for _ in range(2))
+    q, gate = (rng.standard_normal((N, nh, hd)).astype(np.float32) for _ in range(2))
+    bufs = [ctx.put(a) for a in (q, K.view(np.uint16), V.view(np.uint16), np.arange(npages, dtype=np.int32), gate)]
+    out = ctx.alloc(q.nbytes)
+    ctx.gd_attn_batch(*bufs, out, hd, nh, nkv, kv_dim, page, C.c_float(scale), base, N, 1, 0)
+    got = ctx.get(out, q.shape, np.float32)
+    for n in range(0, N, max(1, N // 8)):
+        # ref_attention's scale is 1 / sqrt(hd); the entry's is the f32 nearest 0.07.
+        want = ref_attention(q[n].astype(np.float64) * float(np.float32(scale)) * np.sqrt(hd), K, V, gate[n], nkv,
+                             base + n + 1)
+        assert rel_diff(got[n], want) < 1e-5, n
+    for p in (*bufs, out):
+        ctx.free(p)
+
+
 def test_attention_rejects_bad_shapes(ctx):
     d = ctx.alloc(64)
     lib = ctx.lib
