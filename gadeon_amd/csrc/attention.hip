@@ -1202,10 +1202,12 @@ extern "C" int gd_attn_paged(gd_ctx *ctx, const float *q, const uint16_t *k_cach
     const int cus = ctx->num_cus > 0 ? ctx->num_cus : 256;
     const int blocks = (T - lo + 31) / 32;
     int ns = std::max(1, std::min({blocks, MAX_SPLITS, std::max(DSPLIT, 2 * cus / groups)}));
-    if (ns > DSPLIT &&
-        (!ctx->attn_scratch || (size_t)n_head * ns * (hd + 2) * sizeof(float) > GD_ATTN_SCRATCH_BYTES))
+    if (ns > DSPLIT && (size_t)n_head * ns * (hd + 2) * sizeof(float) > GD_ATTN_SCRATCH_BYTES) ns = DSPLIT;
+    float *pt = ns > DSPLIT ? gd_attn_scratch(ctx) : part;
+    if (!pt) {
         ns = DSPLIT;
-    float *pt = ns > DSPLIT ? ctx->attn_scratch : part;
+        pt = part;
+    }
 #define GD_PAGED(HD_) \
     hipLaunchKernelGGL(k_attn_paged<HD_>, dim3(groups, ns), dim3(64 * PW), 0, ctx->stream, q, k_cache, \
                        v_cache, page_table, T, lo, pt, ns, n_head, n_head_kv, page_size, scale); \
@@ -1246,13 +1248,13 @@ extern "C" int gd_attn_batch(gd_ctx *ctx, const float *q, const uint16_t *k_cach
     const int64_t units = (int64_t)n_head * gd_blocks(N, AQ), row = (int64_t)N * n_head * (hd * 4 + 8);
     const int cus = ctx->num_cus > 0 ? ctx->num_cus : 256;
     int64_t nz = hd != 256 ? 0 : std::min({(int64_t)MAX_KEY_SPLITS, 2 * (int64_t)cus / units, keys / SPLIT_KEYS,
-                           ctx->attn_scratch ? (int64_t)GD_ATTN_SCRATCH_BYTES / row : 0});
-    if (nz > 1) {
+                           (int64_t)GD_ATTN_SCRATCH_BYTES / row});
+    float *scratch = nz > 1 ? gd_attn_scratch(ctx) : nullptr;
+    if (scratch) {
         const int64_t ck = ((keys + nz - 1) / nz + 63) / 64 * 64;
         nz = (keys + ck - 1) / ck;
         const AttnQ qsrc{q, gated ? gate : q, (int64_t)n_head * hd, hd, nullptr, nullptr, 0, 0, 0.f, 0.f};
-        const AttnSplit split{ctx->attn_scratch, (float2 *)(ctx->attn_scratch + nz * N * n_head * hd), (int)nz,
-                              (int)ck};
+        const AttnSplit split{scratch, (float2 *)(scratch + nz * N * n_head * hd), (int)nz, (int)ck};
         const dim3 grid((unsigned)n_head, gd_blocks(N, AQ), (unsigned)nz);
         hipLaunchKernelGGL((k_attn_prefill<256, float, true>), grid, dim3(256), 0, ctx->stream, qsrc, split,
                            k_cache, v_cache, page_table, nullptr, base_pos, out, n_head, n_head_kv, (int)N,

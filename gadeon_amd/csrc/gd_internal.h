@@ -12,25 +12,44 @@
 
 #include "../../include/gadeon_hip.h"
 
+// Device memory that a context and the graphs recorded on it may share: freed
+// by the last that drops it.
+struct gd_buf {
+    void *p = nullptr;
+    std::atomic<int> refs{1};
+};
+// A buffer of `bytes` on the current device, null if the allocation failed; it
+// may be made while a stream is captured (gd_graph_begin).
+gd_buf *gd_buf_new(size_t bytes);
+void gd_buf_drop(gd_buf *b);
+
 struct gd_ctx {
     int device = 0;
     hipStream_t stream = nullptr;
     hipEvent_t ev_start = nullptr;
     hipEvent_t ev_stop = nullptr;
     int num_cus = 0;
-    void *ws = nullptr;          // grow-only workspace (chunked GDN prefill)
+    gd_buf *ws = nullptr;        // grow-only workspace (chunked GDN prefill, GEMM)
     size_t ws_bytes = 0;
     // This device's copy of the allocation-free prefill's scratch array
     // (hipGetSymbolAddress at context creation; null if that failed).
     void *prefill_scratch = nullptr;
-    // Key-split partials of gd_attn_paged beyond the 16 per head its caller's
-    // scratch holds: GD_ATTN_SCRATCH_BYTES, held by the context so that the
-    // entry allocates nothing (it may be recorded); null if that failed.
-    float *attn_scratch = nullptr;
+    // Key-split partials of gd_attn_paged (beyond the 16 per head its caller's
+    // scratch holds) and of gd_attn_batch: GD_ATTN_SCRATCH_BYTES, null if that
+    // failed; reached through gd_attn_scratch.
+    gd_buf *attn = nullptr;
+    // Inside a recording (gd_graph_begin .. gd_graph_end): what the graph will
+    // hold, the workspace if an entry used it and attention partials of its own,
+    // since it may be launched beside this context's calls and outlive them.
+    bool recording = false;
+    gd_buf *rec_ws = nullptr, *rec_attn = nullptr;
     std::string err;
 };
 
 constexpr size_t GD_ATTN_SCRATCH_BYTES = 8u << 20;
+// The attention entries' partials, the context's or the recording's; null if
+// there is no memory for them.
+float *gd_attn_scratch(gd_ctx *ctx);
 
 // Look up this device's address of the prefill scratch array (device current).
 int gd_prefill_scratch_attach(gd_ctx *ctx);

@@ -6,6 +6,7 @@
 #include <stdarg.h>
 #include <string.h>
 #include <mutex>
+#include <new>
 
 static std::mutex g_err_mu;
 static std::string g_err;   // last gd_ctx_create failure (no context yet)
@@ -66,11 +67,8 @@ extern "C" int gd_ctx_create(int device, gd_ctx **out) {
     // needs it, and it reports the failure then.
     (void)gd_prefill_scratch_attach(c);
     // Likewise the attention partials: without them gd_attn_paged splits the
-    // keys no further than its caller's scratch allows.
-    if (hipMalloc((void **)&c->attn_scratch, GD_ATTN_SCRATCH_BYTES) != hipSuccess) {
-        c->attn_scratch = nullptr;
-        (void)hipGetLastError();
-    }
+    // keys no further than its caller's scratch allows, and gd_attn_batch not.
+    c->attn = gd_buf_new(GD_ATTN_SCRATCH_BYTES);
     c->err.clear();
     *out = c;
     return GD_OK;
@@ -82,8 +80,7 @@ extern "C" void gd_ctx_destroy(gd_ctx *ctx) {
     if (ctx->stream) (void)hipStreamSynchronize(ctx->stream);
     if (ctx->ev_start) (void)hipEventDestroy(ctx->ev_start);
     if (ctx->ev_stop) (void)hipEventDestroy(ctx->ev_stop);
-    if (ctx->ws) (void)hipFree(ctx->ws);
-    if (ctx->attn_scratch) (void)hipFree(ctx->attn_scratch);
+    for (gd_buf *b : {ctx->ws, ctx->attn, ctx->rec_ws, ctx->rec_attn}) gd_buf_drop(b);
     if (ctx->stream) (void)hipStreamDestroy(ctx->stream);
     delete ctx;
 }
@@ -96,23 +93,54 @@ extern "C" const char *gd_last_error(const gd_ctx *ctx) {
     return copy.c_str();
 }
 
+// Allocations and frees while this thread captures a stream are refused unless
+// its capture mode is relaxed; neither is part of what is captured.
+static void set_capture_mode(hipStreamCaptureMode &mode) { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+
+gd_buf *gd_buf_new(size_t bytes) {
+    gd_buf *b = new (std::nothrow) gd_buf();
+    if (!b) return nullptr;
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    set_capture_mode(mode);
+    const hipError_t e = hipMalloc(&b->p, bytes);
+    set_capture_mode(mode);
+    if (e == hipSuccess) return b;
+    (void)hipGetLastError();
+    delete b;
+    return nullptr;
+}
+
+void gd_buf_drop(gd_buf *b) {
+    if (!b || b->refs.fetch_sub(1) != 1) return;
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    set_capture_mode(mode);
+    (void)hipFree(b->p);
+    set_capture_mode(mode);
+    delete b;
+}
+
 int gd_ctx_workspace(gd_ctx *ctx, size_t bytes, void **out) {
     if (ctx->ws_bytes < bytes) {
-        if (ctx->ws) {
-            GD_HIP(ctx, hipStreamSynchronize(ctx->stream));
-            GD_HIP(ctx, hipFree(ctx->ws));
-            ctx->ws = nullptr;
-            ctx->ws_bytes = 0;
-        }
-        hipError_t e = hipMalloc(&ctx->ws, bytes);
-        if (e != hipSuccess) {
-            ctx->ws = nullptr;
-            return gd_fail(ctx, GD_ENOMEM, "workspace (%zu bytes): %s", bytes, hipGetErrorString(e));
-        }
+        // Inside a recording this fails, and the recording with it.
+        if (ctx->ws || ctx->recording) GD_HIP(ctx, hipStreamSynchronize(ctx->stream));
+        gd_buf_drop(ctx->ws);
+        ctx->ws_bytes = 0;
+        ctx->ws = gd_buf_new(bytes);
+        if (!ctx->ws) return gd_fail(ctx, GD_ENOMEM, "workspace (%zu bytes): out of memory", bytes);
         ctx->ws_bytes = bytes;
     }
-    *out = ctx->ws;
+    if (ctx->recording && !ctx->rec_ws) {
+        ctx->ws->refs++;
+        ctx->rec_ws = ctx->ws;
+    }
+    *out = ctx->ws->p;
     return GD_OK;
+}
+
+float *gd_attn_scratch(gd_ctx *ctx) {
+    if (!ctx->recording) return ctx->attn ? (float *)ctx->attn->p : nullptr;
+    if (!ctx->rec_attn) ctx->rec_attn = gd_buf_new(GD_ATTN_SCRATCH_BYTES);
+    return ctx->rec_attn ? (float *)ctx->rec_attn->p : nullptr;
 }
 
 extern "C" int gd_alloc(gd_ctx *ctx, size_t bytes, void **dptr) {
@@ -232,34 +260,37 @@ extern "C" int gd_timer_stop(gd_ctx *ctx, float *ms) {
 struct gd_graph {
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
+    gd_buf *ws = nullptr, *attn = nullptr;   // device memory its kernels use
 };
 
 extern "C" int gd_graph_begin(gd_ctx *ctx) {
     GD_CHECK_CTX(ctx);
     GD_HIP(ctx, hipStreamBeginCapture(ctx->stream, hipStreamCaptureModeThreadLocal));
+    ctx->recording = true;
     return GD_OK;
 }
 
 extern "C" int gd_graph_end(gd_ctx *ctx, gd_graph **out) {
     GD_CHECK_CTX(ctx);
     if (out) *out = nullptr;
-    hipGraph_t graph = nullptr;
-    const hipError_t e = hipStreamEndCapture(ctx->stream, &graph);
+    gd_graph *g = new gd_graph();
+    std::swap(g->ws, ctx->rec_ws);
+    std::swap(g->attn, ctx->rec_attn);
+    ctx->recording = false;
+    hipError_t e = hipStreamEndCapture(ctx->stream, &g->graph);
     if (e != hipSuccess) {
-        if (graph) (void)hipGraphDestroy(graph);
+        gd_graph_destroy(g);
         return gd_hip_fail(ctx, e, "gd_graph_end: hipStreamEndCapture");
     }
     if (!out) {
-        (void)hipGraphDestroy(graph);
+        gd_graph_destroy(g);
         return gd_fail(ctx, GD_EINVAL, "gd_graph_end: null out pointer (capture discarded)");
     }
-    gd_graph *g = new gd_graph();
-    g->graph = graph;
-    const hipError_t ei = hipGraphInstantiate(&g->exec, graph, nullptr, nullptr, 0);
-    if (ei != hipSuccess) {
-        (void)hipGraphDestroy(graph);
-        delete g;
-        return gd_hip_fail(ctx, ei, "gd_graph_end: hipGraphInstantiate");
+    e = hipGraphInstantiate(&g->exec, g->graph, nullptr, nullptr, 0);
+    if (e != hipSuccess) {
+        g->exec = nullptr;
+        gd_graph_destroy(g);
+        return gd_hip_fail(ctx, e, "gd_graph_end: hipGraphInstantiate");
     }
     *out = g;
     return GD_OK;
@@ -276,6 +307,8 @@ extern "C" void gd_graph_destroy(gd_graph *g) {
     if (!g) return;
     if (g->exec) (void)hipGraphExecDestroy(g->exec);
     if (g->graph) (void)hipGraphDestroy(g->graph);
+    gd_buf_drop(g->ws);
+    gd_buf_drop(g->attn);
     delete g;
 }
 

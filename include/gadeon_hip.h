@@ -15,7 +15,8 @@
  *     on that context.  (Reference: MetalErr, MetalContext.swift:331-349, and
  *     the non-throwing dispatch methods of MetalEnc.swift:9-13.)
  *   - Device pointers are plain `void*` from gd_alloc.  The caller owns every
- *     device buffer; the context owns only its stream and events.
+ *     device buffer; the context owns its stream and events, a workspace that
+ *     grows with the largest call, and 8 MiB of attention partials.
  *   - Compute entries enqueue on the context stream and return immediately;
  *     gd_sync / gd_download block.  One context must not be used from two
  *     threads at once (MetalBackend.swift:3-4: the session serializes calls).
@@ -101,7 +102,12 @@ int gd_timer_stop(gd_ctx *ctx, float *ms);
  * recorded: no gd_sync, gd_download, gd_upload, gd_alloc/free or timer calls,
  * and no entry that has to grow the context workspace (run it once before
  * recording).  A failing entry inside a recording leaves the capture open;
- * gd_graph_end then fails and discards it. */
+ * gd_graph_end then fails and discards it.  A graph holds the workspace its
+ * calls use, shared with the context's other calls, and attention partials of
+ * its own (8 MiB, where it records gd_attn_paged or gd_attn_batch), until it is
+ * destroyed: it may outlive its context, and be launched on another one as
+ * long as the workspace of the first is not in use at the same time (which GEMMs
+ * of f32 rows or split K and gd_gdn_prefill do). */
 typedef struct gd_graph gd_graph;
 int gd_graph_begin(gd_ctx *ctx);
 int gd_graph_end(gd_ctx *ctx, gd_graph **out);

@@ -248,6 +248,58 @@ def test_prefill_attention_scales(ctx, nh, nkv, N, base):
         ctx.free(p)
 
 
+def test_recorded_calls_hold_their_memory(ctx):
+    """A recording's attention partials are its own and the workspace it used
+    stays with it: launched on another context, between that context's own
+    calls, after its first context has grown its workspace and is gone, every
+    replay of a long-context token, a few-queries prompt and a GEMM of f32 rows
+    gives the direct calls' bits."""
+    hd, nh, nkv, page, T, N, K, R = 256, 8, 2, 16, 4000, 5, 1024, 512
+    rng = np.random.default_rng(3)
+    kv_dim, npages = hd * nkv, T // page + 1
+    f32 = lambda *s: rng.standard_normal(s).astype(np.float32)
+    kc, vc = (ctx.put(f32(npages, page, nkv, hd).astype(np.float16).view(np.uint16)) for _ in range(2))
+    q, gate, other, X = (ctx.put(f32(*s)) for s in ((N, nh, hd), (N, nh, hd), (N, nh, hd), (64, K)))
+    table = ctx.put(rng.permutation(npages).astype(np.int32))
+    w = ga.Q2W()
+    blocks = O.lcg_q2_0(K, R, 9)
+    ctx.gd_q2_0_upload(blocks.ctypes.data, K, R, C.byref(w))
+    outs = [(ctx.alloc(4 * n), n) for n in (nh * hd, N * nh * hd, 8 * R)]
+    part, spare = ctx.alloc(nh * 16 * (hd + 2) * 4), ctx.alloc(N * nh * hd * 4)
+    ctx.sync()
+
+    def attend(c, src, o1, o2):
+        c.gd_attn_paged(src, kc, vc, table, gate, o1, part, hd, nh, nkv, T, kv_dim, page, C.c_float(1 / 16), 1, 0)
+        c.gd_attn_batch(src, kc, vc, table, gate, o2, hd, nh, nkv, kv_dim, page, C.c_float(1 / 16), T - N, N, 1, 0)
+
+    def calls(c):
+        attend(c, q, outs[0][0], outs[1][0])
+        c.gd_q2_0_gemm(C.byref(w), 8, X, ga.F32, outs[2][0], ga.F32)
+
+    first, g = ga.Context(0), C.c_void_p()
+    calls(first)
+    want = [first.get(p, n, np.float32) for p, n in outs]
+    first.gd_graph_begin()
+    calls(first)
+    first.gd_graph_end(C.byref(g))
+    attend(first, other, spare, spare)
+    big = first.alloc(64 * R * 4)
+    first.gd_q2_0_gemm(C.byref(w), 64, X, ga.F32, big, ga.F32)
+    first.close()
+    for _ in range(3):
+        for p, n in outs:
+            ctx.gd_fill_u32(p, 0, n)
+        attend(ctx, other, spare, spare)
+        ctx.gd_graph_launch(g)
+        attend(ctx, other, spare, spare)
+        for (p, n), ref in zip(outs, want):
+            assert np.array_equal(ctx.get(p, n, np.float32), ref)
+    ctx.lib.gd_graph_destroy(g)
+    ctx.gd_q2w_free(C.byref(w))
+    for p in (kc, vc, q, gate, other, X, table, part, spare, *(p for p, _ in outs)):
+        ctx.free(p)
+
+
 def test_attention_rejects_bad_shapes(ctx):
     d = ctx.alloc(64)
     lib = ctx.lib
