@@ -1032,7 +1032,7 @@ int gemm_run(gd_ctx *ctx, const gd_q2w *w, int64_t T, const void *X, int x_dtype
                    "gd_q2_0_gemm_plan: no kernel for mt=%d nt=%d split=%d nw=%d", forced->mt,
                    forced->nt, forced->split, forced->nw);
         p = *forced;
-        const int nblk = p.skinny ? (int)(w->K / 128 + 3) / 4 : (int)(w->K / 128);
+        const int nblk = (int)(w->K / 128);
         const int bps = (nblk + p.split - 1) / p.split;
         p.split = (nblk + bps - 1) / bps;               // splits that hold blocks
     } else {
@@ -1085,7 +1085,7 @@ extern "C" int gd_q2_0_gemm(gd_ctx *ctx, const gd_q2w *w, int64_t T, const void 
 extern "C" int gd_q2_0_gemm_plan(gd_ctx *ctx, const gd_q2w *w, int64_t T, const void *X,
                                  int x_dtype, void *Y, int y_dtype, int mt, int nt, int split,
                                  int nw) {
-    gd_gemm_plan p{mt, nt, split, nw};
+    const gd_gemm_plan p{mt, nt, split, nw};
     return gemm_run(ctx, w, T, X, x_dtype, Y, y_dtype, &p);
 }
 

@@ -287,26 +287,32 @@ def test_gemm_vs_oracle(ctx, T, K, R, xt, yt):
 
 
 @pytest.mark.parametrize("T,K,R", [(32, 640, 100), (31, 1152, 33), (17, 128, 48), (3, 2048, 1),
-                                   (32, 4992, 64), (8, 6144, 3072), (32, 512, 16384), (2, 256, 16416)])
+                                   (32, 4992, 64), (8, 6144, 3072), (17, 6784, 3072), (32, 512, 16384),
+                                   (2, 256, 16416)])
 def test_gemm_few_tokens(ctx, T, K, R):
     """At most 32 tokens, up to the last row count that takes the few-token
     kernel (one round of the CUs) and one past it: K short of whole 512-K
-    chunks, one and several chunks, K splits (6144 x 3072), rows short of a
-    fragment, and (32 | R) the same product with the SwiGLU epilogue.  The
-    f32 products of f16 pairs are exact; a sum of K of them, at any order,
-    stays within K 2^-24 of the sum of their magnitudes."""
+    chunks, one and several chunks, K splits (6144 x 3072: four of three chunks;
+    6784 x 3072: five, the last of two chunks and those of five blocks), rows
+    short of a fragment, and (32 | R) the same product with the SwiGLU
+    epilogue.  Against f64: the f32 products of f16 pairs are exact, and K of
+    them, each partial sum at most about the output's size, round by
+    sqrt(K) 2^-24 of it at 6784 (5e-6): 1e-5 of the largest output.  One
+    product of K lost or doubled is 1e-2 of an output's size."""
     blocks = O.lcg_q2_0(K, R, 5 * K + R)
     w = upload_w(ctx, blocks, K, R)
     Xh = O.lcg_normal_f16(T * K, 83).reshape(T, K)
     Xr = Xh.astype(np.float32)
-    want = np.stack([O.q2_0_matvec(blocks, K, R, Xr[t], threads=8) for t in range(T)])
-    # |w| <= 2 d; d from the blocks' f16 scales.
-    d = np.abs(blocks.reshape(R, K // 128, 34)[:, :, :2].copy().view(np.float16)[..., 0].astype(np.float32))
-    mag = 2 * np.abs(Xr).reshape(T, K // 128, 128).sum(2) @ d.T
+    # (code - 1) d of each weight, in f64.
+    b = blocks.reshape(R, K // 128, 34)
+    d = b[:, :, :2].copy().view(np.float16).astype(np.float64)
+    codes = (b[:, :, 2:, None] >> np.arange(0, 8, 2, dtype=np.uint8)) & 3
+    want = Xr.astype(np.float64) @ ((codes.reshape(R, K // 128, 128) - 1.0) * d).reshape(R, K).T
+    tol = 1e-5 * np.abs(want).max()
     Y = _gemm(ctx, w, Xh.view(np.uint16), ga.F16, ga.F32, T, R)
-    assert np.all(np.abs(Y - want) <= 2 * K * 2.0 ** -24 * mag)
+    assert np.all(np.abs(Y - want) <= tol)
     Y = _gemm(ctx, w, Xr, ga.F32, ga.F16, T, R)
-    assert np.all(np.abs(Y - want) <= 2 * K * 2.0 ** -24 * mag + 2.0 ** -11 * np.abs(want) + 2.0 ** -24)
+    assert np.all(np.abs(Y - want) <= tol + 2.0 ** -11 * np.abs(want) + 2.0 ** -24)
     if R % 32 == 0:
         ff = R // 2
         dX, dO = ctx.put(Xh.view(np.uint16)), ctx.alloc(T * ff * 2)
