@@ -243,7 +243,7 @@ __global__ void gd_rmsnorm_rows_kernel(float *x, int d, int64_t rows, const floa
 
 // Rows of 4 L elements, a row in L lanes' registers (16 bytes a lane) and four
 // rows a thread in flight.  Bound by HBM: 48000 rows of 128 (49 MB) 8.7 us,
-// one row a wave and 4 bytes a lane 14.0.
+// one row a wave and 4 bytes a lane 13.8.
 template <int L>
 __global__ __launch_bounds__(256) void gd_rmsnorm_rows_vec_kernel(float *x, int64_t rows, const float *w, float eps) {
     constexpr int NR = 4, D = 4 * L, G = 256 / L;
@@ -268,8 +268,12 @@ extern "C" int gd_rmsnorm_rows(gd_ctx *ctx, float *x, int d, int64_t rows, const
     GD_CHECK_CTX(ctx);
     GD_REQUIRE(ctx, x && w && d > 0 && rows >= 0, "gd_rmsnorm_rows: bad arguments");
     if (!rows) return GD_OK;
-    // The head dims of the models (14.0 -> 8.7 us, 48000 rows of 128; 16-byte rows).
-    const bool al = (((uintptr_t)x | (uintptr_t)w) & 15) == 0;
+    // The head dims of the models, 16-byte rows, from 2^20 elements on: fewer
+    // leave CUs without a block of 32 (16) rows and pay for its longer chain.  A
+    // chain of calls, rows of 128: 1000 2.2 us (vector kernel 2.8), 6000 3.1
+    // (3.2), 8000 3.4 (3.3), 16000 5.0 (3.9), 48000 13.8 (8.8); rows of 256: 1000
+    // 2.7 (3.0), 4000 3.4 (3.4), 8000 4.5 (4.1).
+    const bool al = (((uintptr_t)x | (uintptr_t)w) & 15) == 0 && rows * d >= 1 << 20;
     if (d == 128 && al)
         hipLaunchKernelGGL(gd_rmsnorm_rows_vec_kernel<32>, dim3(gd_blocks(rows, 32)), dim3(256), 0, ctx->stream, x,
                            rows, w, eps);

@@ -167,6 +167,14 @@ def test_rmsnorm_rows_shapes(ctx, d, rows, off):
         ctx.free(p)
 
 
+@pytest.mark.parametrize("d,rows,off", [(128, 8191, 0), (128, 8192, 0), (128, 8209, 0), (128, 8192, 1),
+                                        (256, 4096, 0), (256, 4111, 0), (256, 4095, 0)])
+def test_rmsnorm_rows_many(ctx, d, rows, off):
+    """Either side of the element count from which a row is 16 bytes a lane,
+    whole and ragged blocks of rows: as test_rmsnorm_rows_shapes."""
+    test_rmsnorm_rows_shapes(ctx, d, rows, off)
+
+
 # ------------------------------------------------------------------ scan
 
 @pytest.mark.parametrize("nV,nK,dS", [(16, 16, 128), (16, 4, 128), (6, 3, 64)])

@@ -54,6 +54,17 @@ def test_conv_few_tokens(ctx, N):
         ctx.free(p)
 
 
+@pytest.mark.parametrize("d,rows", [(128, 64), (128, 1000), (256, 64), (128, 48000)])
+def test_rmsnorm_rows_few(ctx, d, rows):
+    """Few rows, and many, against the kernel for any alignment (x one float off)."""
+    x, w = zeros(ctx, rows * d * 4 + 16), zeros(ctx, d * 4)
+    picked = chain_ms(ctx, lambda: ctx.gd_rmsnorm_rows(x, d, rows, w, EPS))
+    general = chain_ms(ctx, lambda: ctx.gd_rmsnorm_rows(x + 4, d, rows, w, EPS))
+    assert picked < SLACK * general
+    for p in (x, w):
+        ctx.free(p)
+
+
 @pytest.mark.parametrize("n,rows", [(64, 20000), (128, 4000), (512, 20000), (1024, 20000)])
 def test_rmsnorm_short_rows(ctx, n, rows):
     """Many short rows against the kernel for any alignment (x one float off)."""
