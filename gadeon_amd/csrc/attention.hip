@@ -1159,6 +1159,32 @@ int check_attn(gd_ctx *ctx, const char *fn, int hd, int n_head, int n_head_kv, i
 
 }  // namespace
 
+// Most keys that gd_attn_paged gives a wave each of k_attn_decode, in head dims.
+// Where a wave of k_attn_paged has one block (its q's operand, score tiles and
+// merge are then most of its time) that is faster; how far beyond, lies in what
+// the two share out: k_attn_decode 16 workgroups a q head, alike until they are
+// more than the CUs, k_attn_paged the keys of a kv head among its q heads (none
+// to share with one), in registers that leave a wave of head dim 256 half its
+// SIMD.  Crossings of the two, timed in chains of append and attend, in head
+// dims: head dim 128, up to 16 heads 8-10, 24 and 32 heads 6-7 (one kv head for
+// each 8-9), 40 / 8 4, 64 / 8 3 (40 / 40 and 64 / 64 11); head dim 256, 8 heads
+// 7-9 (8 / 8 16), 16 / 4 4.5, 16 / 2 7, 10 / 5, 12 / 6 and 16 / 8 14-15, 24 / 4,
+// 24 / 8 and 32 / 8 3, 24 / 12 and 32 / 16 4-5, 12 / 12 to 64 / 64 from 16 to
+// never.  Times at 24 / 4 x 256: 1152 keys 15.5 us (k_attn_paged 13.3), 3000
+// 23.3 (15.4), 7000 39 (18); 16 / 8 x 128: 577 keys 8.7 (9.6), 1300 11.8 (10.7),
+// 4000 20.3 (12.9); 8 / 8 x 256: 1153 keys 10.5 (14.0), 4000 17.6 (17.5), 7000
+// 23.9 (21.3).
+static int few_keys(const gd_ctx *ctx, int hd, int n_head, int n_head_kv) {
+    const int cus = ctx->num_cus > 0 ? ctx->num_cus : 256;
+    const int wgs = DSPLIT * n_head, G = n_head / n_head_kv;
+    int half;                                             // half head dims
+    if (hd == 128) half = G == 1 || wgs <= cus ? 18 : wgs <= 2 * cus ? 12 : 9;
+    else if (G == 1) half = 2 * wgs <= cus ? 32 : 64;
+    else if (wgs <= cus) half = 2 * wgs <= cus ? 16 : G == 2 ? 28 : 10;
+    else half = 9;
+    return half * (hd / 2);
+}
+
 extern "C" int gd_attn_paged(gd_ctx *ctx, const float *q, const uint16_t *k_cache,
                              const uint16_t *v_cache, const int32_t *page_table,
                              const float *gate, float *out, float *part, int hd, int n_head,
@@ -1170,17 +1196,10 @@ extern "C" int gd_attn_paged(gd_ctx *ctx, const float *q, const uint16_t *k_cach
     int rc = check_attn(ctx, "gd_attn_paged", hd, n_head, n_head_kv, kv_dim, page_size, gated, gate);
     if (rc) return rc;
     GD_REQUIRE(ctx, T > 0 && lo >= 0 && lo < T, "gd_attn_paged: keys [lo=%d, T=%d) empty", lo, T);
-    // Few keys: a wave a key and q head.  Where a wave of k_attn_paged has one
-    // block (its q's operand, score tiles and merge are then most of its time)
-    // that is as fast or faster.  Call times, 24 / 4 heads x 256: 256, 732 and
-    // 1026 keys 8.4, 9.3 and 10.3 us (k_attn_paged 11.3, 11.7 and 10.8), 1536
-    // 14.1 (12.0), 4096 25.8 (13.0); 40 / 8 x 128: 256 keys 7.5 (8.2), 732 9.7
-    // (8.4), 1536 14.0 (9.8), 4096 28.4 (10.8); 16 / 8 x 128: 256 keys 7.7 (8.0),
-    // 732 8.0 (8.3), 1536 9.7 (9.1), 4096 18.5 (9.9).
-    // Inputs off 16-byte alignment, which k_attn_paged loads q, K and V by, take
-    // it at any length.
+    // Few keys, and inputs off 16-byte alignment, which k_attn_paged loads q, K
+    // and V by: a wave a key and q head.
     const bool aligned = ((uintptr_t)q | (uintptr_t)k_cache | (uintptr_t)v_cache) % 16 == 0;
-    if (!aligned || 2 * (int64_t)(T - lo) <= 9 * hd) {
+    if (!aligned || T - lo <= few_keys(ctx, hd, n_head, n_head_kv)) {
         const dim3 grid((unsigned)n_head, DSPLIT);
         uint16_t *kc = const_cast<uint16_t *>(k_cache), *vc = const_cast<uint16_t *>(v_cache);
 #define GD_DECODE(HD_) \

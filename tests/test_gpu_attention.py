@@ -166,6 +166,16 @@ def test_decode_attention_key_blocks(ctx, hd, nh, nkv, page, T, lo):
         ctx.free(p)
 
 
+@pytest.mark.parametrize("hd,nh,nkv,page,T,lo", [
+    (128, 24, 4, 16, 768, 0), (128, 24, 4, 16, 769, 0), (128, 6, 6, 16, 1153, 0), (128, 34, 2, 16, 577, 0),
+    (256, 24, 4, 16, 1153, 0), (256, 24, 4, 16, 1152, 0), (256, 12, 6, 16, 3585, 0), (256, 12, 4, 5, 1300, 19),
+    (256, 3, 1, 16, 2050, 1), (256, 9, 9, 16, 8193, 0), (256, 5, 5, 16, 4097, 0)])
+def test_decode_attention_last_few_keys(ctx, hd, nh, nkv, page, T, lo):
+    """The last key count that goes a wave a key and the first that does not,
+    by the heads and what they share: as test_decode_attention_key_blocks."""
+    test_decode_attention_key_blocks(ctx, hd, nh, nkv, page, T, lo)
+
+
 @pytest.mark.parametrize("hd,nh,nkv", [(128, 10, 2), (256, 6, 1)])
 @pytest.mark.parametrize("off", [(4, 0, 0), (0, 4, 0), (0, 0, 4), (8, 8, 8), (0, 0, 0)])
 def test_decode_attention_alignment(ctx, hd, nh, nkv, off):

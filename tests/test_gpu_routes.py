@@ -86,3 +86,20 @@ def test_rmsnorm_many_rows(ctx):
         assert np.allclose(ctx.get(x + r * n * 4, n, np.float32), 1, rtol=1e-6)
     for p in (x, w):
         ctx.free(p)
+
+
+@pytest.mark.parametrize("hd,nh,nkv,T", [(256, 8, 8, 1153), (256, 8, 8, 3000), (128, 16, 8, 577), (128, 16, 16, 640),
+                                         (256, 24, 4, 9000), (256, 16, 16, 3000)])
+def test_decode_attention_keys(ctx, hd, nh, nkv, T):
+    """Few heads, or one a kv head, over middling contexts, and the usual long
+    one, against the wave-a-key kernel, which a q off 16-byte alignment takes."""
+    page, kv_dim = 16, nkv * hd
+    npages = -(-T // page)
+    kc, vc = (zeros(ctx, npages * page * kv_dim * 2) for _ in range(2))
+    table = ctx.put(np.arange(npages, dtype=np.int32))
+    q, gate, out, part = (zeros(ctx, n * 4 + 16) for n in (nh * hd, nh * hd, nh * hd, nh * 16 * (hd + 2)))
+    call = lambda x: ctx.gd_attn_paged(x, kc, vc, table, gate, out, part, hd, nh, nkv, T, kv_dim, page,
+                                       C.c_float(hd ** -0.5), 1, 0)
+    assert chain_ms(ctx, lambda: call(q)) < SLACK * chain_ms(ctx, lambda: call(q + 4))
+    for p in (kc, vc, table, q, gate, out, part):
+        ctx.free(p)
