@@ -1255,18 +1255,20 @@ extern "C" int gd_attn_batch(gd_ctx *ctx, const float *q, const uint16_t *k_cach
     if (!N) return GD_OK;
     // Few queries over many keys leave most of the chip idle, each block a
     // serial chain over all keys, 2.2 us per 32 of them at head dim 256: the
-    // keys are split, for up to two blocks a CU and what the context's scratch
-    // holds, from 64 keys a split (about what the partials' round trip and the
-    // combine cost).  24 / 4 x 256, 16 queries after 112 keys 22.4 -> 15.7 us,
-    // 500 50.3 -> 21.6, 4000 288 -> 51; 100 after 4000 295 -> 109; 200 after
-    // none 29.7, unsplit (the chip is filled from 11 query blocks on).
+    // keys are split, for one block a CU (its registers leave no room for a
+    // second; two rounds of half the keys 53 us for 47 below, 16 / 4 heads 53 for
+    // 37) and what the scratch holds, from 64 keys a split (about what the
+    // partials' round trip and the combine cost).  Append and attend, 24 / 4 x
+    // 256, 16 queries after 200 keys 21.9 us, 1000 25.4, 4000 47 (unsplit 288);
+    // 100 after 4000 112 (295), 150 159; from about 170 queries at 24 heads the
+    // scratch holds no two splits: 250 after 4000 309, as unsplit.
     //   Head dim 128 stays unsplit: which of its q halves belong to two roundings
     // (k_attn_prefill) depends on the compiled variant, and outputs would differ
     // between a split and an unsplit call by up to 7e-4 of their size.
     const int64_t keys = (int64_t)base_pos + N;
     const int64_t units = (int64_t)n_head * gd_blocks(N, AQ), row = (int64_t)N * n_head * (hd * 4 + 8);
     const int cus = ctx->num_cus > 0 ? ctx->num_cus : 256;
-    int64_t nz = hd != 256 ? 0 : std::min({(int64_t)MAX_KEY_SPLITS, 2 * (int64_t)cus / units, keys / SPLIT_KEYS,
+    int64_t nz = hd != 256 ? 0 : std::min({(int64_t)MAX_KEY_SPLITS, (int64_t)cus / units, keys / SPLIT_KEYS,
                            (int64_t)GD_ATTN_SCRATCH_BYTES / row});
     float *scratch = nz > 1 ? gd_attn_scratch(ctx) : nullptr;
     if (scratch) {
