@@ -763,6 +763,9 @@ double round_cost(const Shape &sh, int64_t units, int cus, int bps) {
 // 32 x 12288 x 12288 21.7 -> 20.4, 32 x 512 x 512 5.9 -> 3.6.  In a second
 // round the tiles draw level (27 x 5120 x 17408: 16.6, skinny 17.3) and ahead
 // (20 x 5120 x 98304: 51.2, skinny 52.7; 3 x 128 x 70000: 3.6, skinny 9.2).
+// A chunk is 512 K whatever K holds: up to 384 a 32-token tile of 128 rows over
+// all of K is done first (chains of calls, 8 x K x 8224, K = 128, 256 and 384:
+// 2.55, 2.9 and 3.3 us; skinny 3.65 each; two tiles a wave 2.9, 3.4, 3.9).
 // Its K is split while the splits fit the round and save more chunks, at
 // 0.65 us each, than the reduction's launch and traffic cost.
 gd_gemm_plan gd_gemm_choose(gd_ctx *ctx, int64_t T, int64_t K, int64_t R, int x_dtype) {
@@ -775,6 +778,7 @@ gd_gemm_plan gd_gemm_choose(gd_ctx *ctx, int64_t T, int64_t K, int64_t R, int x_
     const int cus = ctx->num_cus > 0 ? ctx->num_cus : 256;
     const int64_t skinny_wgs = (R + 32 * SK_FRAGS - 1) / (32 * SK_FRAGS);
     if (T <= 32 && skinny_wgs <= cus) {
+        if (K <= 384) return gd_gemm_plan{1, 1, 1, 4};
         const int chunks = (int)((K + SK_K - 1) / SK_K);
         gd_gemm_plan best{1, 1, 1, 4, 0, 1};
         double best_cost = 1e30;
@@ -919,10 +923,16 @@ int gd_gemm_glu(gd_ctx *ctx, const gd_q2w *w, int64_t T, const void *X, uint16_t
     GD_REQUIRE(ctx, (uint64_t)(R / 32 + 2) * (uint64_t)((nblk + 3) / 4) * 2048u < (1ULL << 32),
                "gd_gemm_glu: K=%d R=%d spans 4 GiB of codes in one buffer resource", K, R);
     const int cus = ctx->num_cus > 0 ? ctx->num_cus : 256;
-    // Few tokens: 27 x 5120, ff 17408 34.5 -> 26.8 us (weights from HBM), 16 x
-    // 4096, ff 12288 18.6 -> 12.8, 32 x 2048, ff 6144 10.8 -> 6.0, 7 x 384, ff
-    // 48 4.5 -> 4.2.  A forced tile plan stays with the tiles.
-    if (T <= 32 && tile17 < 0) return launch_skinny(ctx, w, T, X, out, 1, ff / 16, 1, ff);
+    // Few tokens: in one round of its workgroups (32 columns) the few-token kernel
+    // from K = 384 on (8 tokens, ff 8192: K = 256 3.9 us, tiles 3.7; 384 3.9, 4.2;
+    // 2048 5.7, 10.6; 5120 9.6, 22.7), in up to three, where the tiles' units still
+    // pass in one or two, from 1024 on (ff 17408: 640 8.5, 6.5; 1024 8.5, 8.5; 2048
+    // 11.7, 14.3; 5120 21.0, 30.7).  Beyond the tiles are ahead (ff 34816: 384 9.7,
+    // 5.3; 2048 18.1, 14.6; 5120 32.2, 31.1) or level (70000 x 2048).  A forced
+    // tile plan stays with the tiles.
+    const int64_t sk_wgs = gd_blocks(ff / 16, SK_FRAGS);
+    if (T <= 32 && tile17 < 0 && (sk_wgs <= cus ? K >= 384 : sk_wgs <= 3 * (int64_t)cus && K >= 1024))
+        return launch_skinny(ctx, w, T, X, out, 1, ff / 16, 1, ff);
     auto cols = [](const Shape &sh) { return 16 * sh.nw * sh.nt; };
     auto tiles_t = [&](const Shape &sh) { return (T + sh.mt * 32 - 1) / (sh.mt * 32); };
     // One launch of tile sh over ncols columns, K split into nz parts (the

@@ -288,14 +288,15 @@ def test_gemm_vs_oracle(ctx, T, K, R, xt, yt):
 
 @pytest.mark.parametrize("T,K,R", [(32, 640, 100), (31, 1152, 33), (17, 128, 48), (3, 2048, 1),
                                    (32, 4992, 64), (8, 6144, 3072), (17, 6784, 3072), (32, 512, 16384),
-                                   (2, 256, 16416)])
+                                   (2, 256, 16416), (17, 384, 8224), (17, 512, 8224), (5, 384, 16384),
+                                   (5, 384, 16416), (3, 1024, 49152), (3, 1024, 49184), (2, 896, 32768)])
 def test_gemm_few_tokens(ctx, T, K, R):
     """At most 32 tokens, up to the last row count that takes the few-token
-    kernel (one round of the CUs) and one past it: K short of whole 512-K
-    chunks, one and several chunks, K splits (6144 x 3072: four of three chunks;
-    6784 x 3072: five, the last of two chunks and those of five blocks), rows
-    short of a fragment, and (32 | R) the same product with the SwiGLU
-    epilogue.  Against f64: the f32 products of f16 pairs are exact, and K of
+    kernel (one round of the CUs, three for the SwiGLU product of long K) and one
+    past it, and the longest K that does not: K short of whole 512-K chunks, one
+    and several chunks, K splits (6144 x 3072: four of three chunks; 6784 x 3072:
+    five, the last of two chunks and those of five blocks), rows short of a
+    fragment, and (32 | R) the same product with the SwiGLU epilogue.  Against f64: the f32 products of f16 pairs are exact, and K of
     them, each partial sum at most about the output's size, round by
     sqrt(K) 2^-24 of it at 6784 (5e-6): 1e-5 of the largest output.  One
     product of K lost or doubled is 1e-2 of an output's size."""

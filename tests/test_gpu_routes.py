@@ -103,3 +103,35 @@ def test_decode_attention_keys(ctx, hd, nh, nkv, T):
     assert chain_ms(ctx, lambda: call(q)) < SLACK * chain_ms(ctx, lambda: call(q + 4))
     for p in (kc, vc, table, q, gate, out, part):
         ctx.free(p)
+
+
+def weights(ctx, K, R):
+    w = ga.Q2W()
+    ctx.gd_q2w_alloc(K, R, C.byref(w))
+    ctx.gd_rand_q2w(C.byref(w), 5, 0.01, 0.05)
+    return w
+
+
+@pytest.mark.parametrize("T,K,ff", [(2, 128, 17408), (8, 256, 8192), (8, 384, 34816), (17, 640, 12288),
+                                    (32, 1024, 34816), (2, 2048, 34816), (27, 5120, 17408), (32, 2048, 6144)])
+def test_swiglu_few_tokens(ctx, T, K, ff):
+    """Few tokens at every K and ff against the tiles, which a forced plan takes."""
+    w, x, o = weights(ctx, K, 2 * ff), zeros(ctx, T * K * 2), zeros(ctx, T * ff * 2)
+    picked = chain_ms(ctx, lambda: ctx.gd_q2_0_gemm_swiglu(C.byref(w), T, x, o), 20)
+    tiles = chain_ms(ctx, lambda: ctx.gd_q2_0_gemm_swiglu_plan(C.byref(w), T, x, o, 0), 20)
+    assert picked < 1.15 * tiles
+    ctx.gd_q2w_free(C.byref(w))
+    for p in (x, o):
+        ctx.free(p)
+
+
+@pytest.mark.parametrize("T,K,R", [(2, 128, 1024), (8, 128, 12288), (32, 256, 16384), (8, 256, 4096), (17, 384, 16384), (27, 5120, 5120)])
+def test_gemm_few_tokens_plan(ctx, T, K, R):
+    """Few tokens at every K against a tile that needs no K split."""
+    w, x, o = weights(ctx, K, R), zeros(ctx, T * K * 2), zeros(ctx, T * R * 4)
+    picked = chain_ms(ctx, lambda: ctx.gd_q2_0_gemm(C.byref(w), T, x, ga.F16, o, ga.F32), 20)
+    tiles = chain_ms(ctx, lambda: ctx.gd_q2_0_gemm_plan(C.byref(w), T, x, ga.F16, o, ga.F32, 1, 1, 1, 4), 20)
+    assert picked < 1.15 * tiles
+    ctx.gd_q2w_free(C.byref(w))
+    for p in (x, o):
+        ctx.free(p)
