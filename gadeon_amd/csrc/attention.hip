@@ -708,13 +708,23 @@ __global__ __launch_bounds__(2 * HD) void k_attn_decode(
 // (37 MB, each read by six heads' workgroups); this, on the 16 splits of
 // eight waves that the caller's scratch allows, 21 us (64 CUs), on 64 splits of
 // four 13; 32000 keys 27 us (4.9 TB/s of cache).
-//   Against 64 bits (24 / 4 x 256, unit normal q, K, V): 2.1e-7 of the output at
-// 3000 and at 9001 keys, 2.2e-7 at 30000; one wave a key in f32 1.8e-7,
-// 2.2e-7, 3.2e-7.  With unscaled q and weights the low halves fell below
-// f16's normal range (3.4e-7).
+//   Against 64 bits (24 / 4 x 256, unit normal q, K, V): 2.0e-7 of the output at
+// 1200 keys, 2.1e-7 at 3000, 2.3e-7 at 9001, 2.4e-7 at 32768; one wave a key in
+// f32 1.9e-7, 2.0e-7, 2.4e-7, 3.5e-7 (40 / 8 x 128: 1.9, 2.1, 2.2 and 2.4e-7 to
+// 1.9, 2.2, 2.9 and 4.6e-7).  With unscaled q and weights the low halves fell
+// below f16's normal range (3.4e-7); with scaled scores, rounded before the
+// maximum is taken off, it was 3% more.
+//   An infinity of the cache (an append past f16's range) counts as it does in
+// k_attn_decode: a key of score -inf weighs nothing, an infinite V gives its dim
+// that infinity.  For that no weight's high half is zero (0 x inf is NaN; the low
+// half takes the difference back), V past the last key is zero, and what a low
+// half adds to a score or a sum is kept finite.
 constexpr int PW = 4;           // waves
 constexpr int SPLIT_KEYS = 64, MAX_KEY_SPLITS = 32;   // fewest keys of a prefill's split, most splits
 constexpr float LOG2E = 1.4426950408889634f;
+// A low half's sum where the high half's is infinite may be NaN or infinite: -FLT_MAX
+// or FLT_MAX (v_med3 of a NaN is the least of the others).
+__device__ __forceinline__ float finite(float x) { return __builtin_amdgcn_fmed3f(x, -__FLT_MAX__, __FLT_MAX__); }
 template <int HD>
 __global__ __launch_bounds__(64 * PW) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_attn_paged(
         const float *q, const uint16_t *kc, const uint16_t *vc, const int32_t *page_table, int T,
@@ -778,6 +788,7 @@ __global__ __launch_bounds__(64 * PW) __attribute__((amdgpu_waves_per_eu(2, 2)))
         const int ex = min(max((int)(__float_as_uint(mx) >> 23), 40), 254) - 127;
         const float up = __uint_as_float((uint32_t)(127 + 14 - ex) << 23);
         sf = scale * LOG2E * __uint_as_float((uint32_t)(127 - 14 + ex) << 23);
+        if (fabsf(sf) < 0x1p-126f) sf = 0x1p-126f;        // weights of 1 alike; times inf not NaN
 #pragma unroll
         for (int ks = 0; ks < KS; ks++) {
             if (ks % PW != w) continue;
@@ -793,6 +804,7 @@ __global__ __launch_bounds__(64 * PW) __attribute__((amdgpu_waves_per_eu(2, 2)))
     }
     fetchK(sl);
     fetchV(sl);
+    const float none = sf < 0.f ? INFINITY : -INFINITY;   // the score of no key
     f32x4 acc[DT];                                        // O^T rows 16 dt + 4 g + v
 #pragma unroll
     for (int dt = 0; dt < DT; dt++) acc[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -817,21 +829,30 @@ __global__ __launch_bounds__(64 * PW) __attribute__((amdgpu_waves_per_eu(2, 2)))
         __builtin_amdgcn_sched_barrier(0);
         const int s2 = slot_of(j + 2 * step);
         fetchK(sn);
+        if (lo + 32 * j + 32 > T) {                       // past the last key zeros
 #pragma unroll
-        for (int n = 0; n < VCH; n++)
-            *(u32x4 *)&Vs[w][(n * 64 + lane) / CPK][8 * (lane % CPK)] = vreg[n];
+            for (int n = 0; n < VCH; n++) {
+                const int k = (n * 64 + lane) / CPK;
+                *(u32x4 *)&Vs[w][k][8 * (lane % CPK)] = lo + 32 * j + k < T ? vreg[n] : u32x4{0u, 0u, 0u, 0u};
+            }
+        } else {
+#pragma unroll
+            for (int n = 0; n < VCH; n++) *(u32x4 *)&Vs[w][(n * 64 + lane) / CPK][8 * (lane % CPK)] = vreg[n];
+        }
         fetchV(sn);
         sn = s2;
         __builtin_amdgcn_sched_barrier(0);
-        // hi + lo of a head's score; keys 16 kt + 4 g + v of the block.
+        // hi + lo of a head's score; keys 16 kt + 4 g + v of the block.  (Unscaled:
+        // a weight's exponent is rounded once.)
         float bmax = -INFINITY;
 #pragma unroll
         for (int kt = 0; kt < 2; kt++)
 #pragma unroll
             for (int v = 0; v < 4; v++) {
-                sc[kt][v] = (sc[kt][v] + gd_dpp<GD_DPP_ROR8>(sc[kt][v])) * sf;
-                if (lo + 32 * j + 16 * kt + 4 * g + v >= T) sc[kt][v] = -INFINITY;
-                bmax = fmaxf(bmax, sc[kt][v]);
+                const float o = gd_dpp<GD_DPP_ROR8>(sc[kt][v]);
+                sc[kt][v] = (lr < 8 ? sc[kt][v] : o) + finite(lr < 8 ? o : sc[kt][v]);
+                if (lo + 32 * j + 16 * kt + 4 * g + v >= T) sc[kt][v] = none;
+                bmax = fmaxf(bmax, sc[kt][v] * sf);
             }
         bmax = fmaxf(bmax, __shfl_xor(bmax, 16, 64));
         bmax = fmaxf(bmax, __shfl_xor(bmax, 32, 64));
@@ -850,11 +871,12 @@ __global__ __launch_bounds__(64 * PW) __attribute__((amdgpu_waves_per_eu(2, 2)))
         for (int kt = 0; kt < 2; kt++)
 #pragma unroll
             for (int v = 0; v < 4; v++) {
-                const float p = __builtin_amdgcn_exp2f(sc[kt][v] - m) * 16384.f;
-                l += p;
-                f16 hi, lo_;
-                gd_split_f16(p, hi, lo_);
-                pf[4 * kt + v] = lr < 8 ? hi : lo_;
+                const float p = __builtin_amdgcn_exp2f(fmaf(sc[kt][v], sf, -m));
+                l = fmaf(p, 16384.f, l);
+                float ph = fmaf(p, 16384.f, 0x1p-24f);    // never 0
+                asm("" : "+v"(ph));
+                const f16 hi = (f16)ph;
+                pf[4 * kt + v] = lr < 8 ? hi : (f16)fmaf(p, 16384.f, -(float)hi);
             }
         typedef short s16x4 __attribute__((ext_vector_type(4)));
         typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
@@ -883,7 +905,7 @@ __global__ __launch_bounds__(64 * PW) __attribute__((amdgpu_waves_per_eu(2, 2)))
 #pragma unroll
     for (int dt = 0; dt < DT; dt++) {
 #pragma unroll
-        for (int v = 0; v < 4; v++) acc[dt][v] += gd_dpp<GD_DPP_ROR8>(acc[dt][v]);
+        for (int v = 0; v < 4; v++) acc[dt][v] += finite(gd_dpp<GD_DPP_ROR8>(acc[dt][v]));
         if (lr < 8) *(f32x4 *)&red[(w * 8 + lr) * HD + 16 * dt + 4 * g] = acc[dt] * f;
     }
     __syncthreads();
@@ -936,10 +958,10 @@ __global__ __launch_bounds__(512) void k_attn_paged_combine(const float *part, i
     __shared__ float fs[MAX_SPLITS], sum[NR][HD];
     const int h = blockIdx.x, t = threadIdx.x, d = t % HD, r = t / HD;
     const float *p = part + (int64_t)h * ns * (HD + 2);
-    // Past the last split: the last one, at weight zero.
+    // Past the last split, at weight zero: a sum of weights (sums may be infinite).
     float a[MAX_SPLITS / NR];
 #pragma unroll
-    for (int s = 0; s < MAX_SPLITS / NR; s++) a[s] = p[(int64_t)min(r + NR * s, ns - 1) * (HD + 2) + d];
+    for (int s = 0; s < MAX_SPLITS / NR; s++) a[s] = p[r + NR * s < ns ? (r + NR * s) * (HD + 2) + d : HD + 1];
     float inv = 0.f;
     {
         const int lane = t & 63;                          // every wave: the weight of split lane

@@ -207,6 +207,54 @@ def test_decode_attention_alignment(ctx, hd, nh, nkv, off):
         ctx.free(p)
 
 
+@pytest.mark.parametrize("hd,nh,nkv", [(128, 10, 2), (256, 6, 1)])
+@pytest.mark.parametrize("T", [200, 5003])
+def test_decode_attention_infinities(ctx, hd, nh, nkv, T):
+    """Infinite cache entries, with few keys and with many (either kernel): an
+    infinite V, at a middling key, at one of almost no weight (below 1e-9
+    of the largest), at the one key that holds almost all of it (its weight has no
+    low half) and at the last key, gives its dim that infinity and leaves the
+    others; an infinite K gives a key no weight where its score is -inf, and
+    NaN where it is +inf."""
+    page = 16
+    rng = np.random.default_rng(hd + T)
+    kv_dim, npages = hd * nkv, T // page + 1
+    table = rng.permutation(npages).astype(np.int32)
+    K, V = (rng.standard_normal((npages * page, nkv, hd)).astype(np.float16) for _ in range(2))
+    q, gate = (rng.standard_normal((nh, hd)).astype(np.float32) for _ in range(2))
+    q[:, 7] = np.where(np.arange(nh) % 3 == 2, -1.0, 1.0)        # the sign of an infinite K's score
+    grp, sc = nh // nkv, 1 / np.sqrt(hd)
+    for g in range(nkv):                                        # the heavy and the light key
+        u = q[g * grp:(g + 1) * grp].mean(0)
+        u[7] = 0
+        K[150, g], K[90, g] = 12 * u, -6 * u
+    for j, d, x in ((60, 3, np.inf), (90, 4, -np.inf), (150, 5, np.inf), (T - 1, 6, -np.inf)):
+        V[j, :, d] = x
+    K[160, :, 7] = -np.inf
+    paged = np.empty((2, npages, page, nkv, hd), np.float16)
+    paged[:, table] = np.stack([K, V]).reshape(2, npages, page, nkv, hd)
+    bufs = [ctx.put(a) for a in (q, paged[0].view(np.uint16), paged[1].view(np.uint16), table, gate)]
+    out, part = ctx.alloc(nh * hd * 4), ctx.alloc(nh * 16 * (hd + 2) * 4)
+    ctx.gd_attn_paged(*bufs, out, part, hd, nh, nkv, T, kv_dim, page, C.c_float(sc), 1, 0)
+    got = ctx.get(out, (nh, hd), np.float32)
+    Kz, Vz = K.copy(), np.where(np.isinf(V), 0, V)
+    Kz[160, :, 7] = 0
+    for h in range(nh):
+        if q[h, 7] < 0:
+            assert np.isnan(got[h]).all(), h
+            continue
+        s = Kz[:T, h // grp].astype(np.float64) @ q[h].astype(np.float64) * sc
+        s[160] = -np.inf
+        p = np.exp(s - s.max())
+        assert p[150] / p.sum() > 0.5 and p[90] / p[150] < 1e-9       # heavy and light
+        want = (p / p.sum()) @ Vz[:T, h // grp].astype(np.float64) * sigmoid(gate[h].astype(np.float64))
+        assert got[h, 3] == np.inf and got[h, 4] == -np.inf and got[h, 5] == np.inf and got[h, 6] == -np.inf, h
+        fin = np.r_[0:3, 7:hd]
+        assert rel_diff(got[h, fin], want[fin]) < 3e-6, h
+    for p in (*bufs, out, part):
+        ctx.free(p)
+
+
 @pytest.mark.parametrize("hd,nh,nkv,page,N,base", [
     (256, 6, 2, 16, 1, 127), (256, 8, 2, 5, 3, 700), (256, 4, 4, 16, 65, 1000), (256, 4, 1, 16, 200, 0),
     (256, 2, 1, 7, 64, 4100)])
