@@ -2,9 +2,9 @@
 has a second kernel that a call can be put on (an output over its input, a
 start off 16-byte alignment, a forced plan), the one that the rule picks for
 the plain call is not the slower one.  Each side is a recorded chain of calls,
-the fastest of several replays; 1.25 leaves room for the placement of buffers
+the fastest of several replays; 1.15 leaves room for the placement of buffers
 and for the other kernel's own small costs, and the rules that these tests
-were written against were off by 1.3 to 3."""
+were written against were off by 1.2 to 4."""
 import ctypes as C
 
 import numpy as np
@@ -15,7 +15,7 @@ import gadeon_amd as ga
 pytestmark = pytest.mark.gpu
 
 EPS = 1e-6
-SLACK = 1.25
+SLACK = 1.15
 
 
 def chain_ms(ctx, call, n=50, replays=12):
@@ -56,10 +56,10 @@ def test_conv_few_tokens(ctx, N):
 
 @pytest.mark.parametrize("d,rows", [(128, 64), (128, 1000), (256, 64), (128, 48000)])
 def test_rmsnorm_rows_few(ctx, d, rows):
-    """Few rows, and many, against the kernel for any alignment (x one float off)."""
-    x, w = zeros(ctx, rows * d * 4 + 16), zeros(ctx, d * 4)
+    """Few rows, and many, against the kernel for any alignment (w one float off)."""
+    x, w = zeros(ctx, rows * d * 4), zeros(ctx, d * 4 + 16)
     picked = chain_ms(ctx, lambda: ctx.gd_rmsnorm_rows(x, d, rows, w, EPS))
-    general = chain_ms(ctx, lambda: ctx.gd_rmsnorm_rows(x + 4, d, rows, w, EPS))
+    general = chain_ms(ctx, lambda: ctx.gd_rmsnorm_rows(x, d, rows, w + 4, EPS))
     assert picked < SLACK * general
     for p in (x, w):
         ctx.free(p)
@@ -67,10 +67,10 @@ def test_rmsnorm_rows_few(ctx, d, rows):
 
 @pytest.mark.parametrize("n,rows", [(64, 20000), (128, 4000), (512, 20000), (1024, 20000)])
 def test_rmsnorm_short_rows(ctx, n, rows):
-    """Many short rows against the kernel for any alignment (x one float off)."""
-    x, w, y = zeros(ctx, rows * n * 4 + 16), zeros(ctx, n * 4), zeros(ctx, rows * n * 4)
+    """Many short rows against the kernel for any alignment (w one float off)."""
+    x, w, y = zeros(ctx, rows * n * 4), zeros(ctx, n * 4 + 16), zeros(ctx, rows * n * 4)
     picked = chain_ms(ctx, lambda: ctx.gd_rmsnorm(x, w, y, ga.F32, n, rows, EPS), 20)
-    general = chain_ms(ctx, lambda: ctx.gd_rmsnorm(x + 4, w, y, ga.F32, n, rows, EPS), 20)
+    general = chain_ms(ctx, lambda: ctx.gd_rmsnorm(x, w + 4, y, ga.F32, n, rows, EPS), 20)
     assert picked < SLACK * general
     for p in (x, w, y):
         ctx.free(p)
@@ -100,7 +100,8 @@ def test_decode_attention_keys(ctx, hd, nh, nkv, T):
     q, gate, out, part = (zeros(ctx, n * 4 + 16) for n in (nh * hd, nh * hd, nh * hd, nh * 16 * (hd + 2)))
     call = lambda x: ctx.gd_attn_paged(x, kc, vc, table, gate, out, part, hd, nh, nkv, T, kv_dim, page,
                                        C.c_float(hd ** -0.5), 1, 0)
-    assert chain_ms(ctx, lambda: call(q)) < SLACK * chain_ms(ctx, lambda: call(q + 4))
+    picked = chain_ms(ctx, lambda: call(q))
+    assert picked < SLACK * chain_ms(ctx, lambda: call(q + 4))
     for p in (kc, vc, table, q, gate, out, part):
         ctx.free(p)
 
@@ -119,7 +120,7 @@ def test_swiglu_few_tokens(ctx, T, K, ff):
     w, x, o = weights(ctx, K, 2 * ff), zeros(ctx, T * K * 2), zeros(ctx, T * ff * 2)
     picked = chain_ms(ctx, lambda: ctx.gd_q2_0_gemm_swiglu(C.byref(w), T, x, o), 20)
     tiles = chain_ms(ctx, lambda: ctx.gd_q2_0_gemm_swiglu_plan(C.byref(w), T, x, o, 0), 20)
-    assert picked < 1.15 * tiles
+    assert picked < SLACK * tiles
     ctx.gd_q2w_free(C.byref(w))
     for p in (x, o):
         ctx.free(p)
@@ -131,7 +132,7 @@ def test_gemm_few_tokens_plan(ctx, T, K, R):
     w, x, o = weights(ctx, K, R), zeros(ctx, T * K * 2), zeros(ctx, T * R * 4)
     picked = chain_ms(ctx, lambda: ctx.gd_q2_0_gemm(C.byref(w), T, x, ga.F16, o, ga.F32), 20)
     tiles = chain_ms(ctx, lambda: ctx.gd_q2_0_gemm_plan(C.byref(w), T, x, ga.F16, o, ga.F32, 1, 1, 1, 4), 20)
-    assert picked < 1.15 * tiles
+    assert picked < SLACK * tiles
     ctx.gd_q2w_free(C.byref(w))
     for p in (x, o):
         ctx.free(p)
