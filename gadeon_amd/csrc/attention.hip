@@ -264,10 +264,12 @@ __global__ __launch_bounds__(256) void k_attn_prefill(
     // B operand of S^T: q[n][32 ks + 8 g + e] * scale, split hi + lo.  Head dim
     // 128 leaves it to the compiler, which rounds hi from the exact product and
     // lo from its f32 rounding: where those two round to different f16 the halves
-    // are an ulp apart (2^-11 of one dim's share of a score; up to 1.5e-3 of the
-    // rms in single outputs, 2.9e-6 in all).  Callers compare its outputs with
-    // recorded ones more closely than that, so it stays; head dim 256's scale
-    // 1/16 is exact either way, and other scales keep 22 bits.
+    // are an ulp apart (2^-11 of one dim's share of a score).  512 queries after
+    // 3584 keys, 40 / 8 heads, against 64 bits: 3.2e-6 of the output, 6e-4 of its
+    // rms in the worst element; by gd_split_f16 7e-7 and 2e-5, at the same time.
+    // Its outputs are compared with recorded ones at 4e-4 of the rms an element,
+    // less than the two forms differ by, so it stays; head dim 256's scale 1/16 is
+    // exact either way, and its other scales keep 22 bits.
     const int64_t qoff = (int64_t)(valid ? n : N - 1) * qsrc.tstride + (int64_t)h * qsrc.hstride;
     f16x8 qh[HD / 32], ql[HD / 32];
     {
@@ -316,16 +318,21 @@ __global__ __launch_bounds__(256) void k_attn_prefill(
 #pragma unroll
         for (int ks = 0; ks < HD / 32; ks++)
 #pragma unroll
-            for (int e = 0; e < 8; e++) {
-                const float v = x[ks][e] * scale;
+            for (int e = 0; e < 8; e += 2) {
+                const float v[2] = {x[ks][e] * scale, x[ks][e + 1] * scale};
                 if constexpr (HD == 256) {
-                    f16 hi, lo;
-                    gd_split_f16(v, hi, lo);
-                    qh[ks][e] = hi;
-                    ql[ks][e] = lo;
+                    f16x2 hi, lo;
+                    gd_split2_f16(v[0], v[1], hi, lo);
+                    qh[ks][e] = hi[0];
+                    qh[ks][e + 1] = hi[1];
+                    ql[ks][e] = lo[0];
+                    ql[ks][e + 1] = lo[1];
                 } else {
-                    qh[ks][e] = (f16)v;
-                    ql[ks][e] = (f16)(v - (float)qh[ks][e]);
+#pragma unroll
+                    for (int i = 0; i < 2; i++) {
+                        qh[ks][e + i] = (f16)v[i];
+                        ql[ks][e + i] = (f16)(v[i] - (float)qh[ks][e + i]);
+                    }
                 }
             }
     }
