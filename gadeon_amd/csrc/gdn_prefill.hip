@@ -17,9 +17,16 @@
 // MI355X design.  Every product above runs on v_mfma_f32_16x16x32_f16 with
 // f32 accumulation.  Operands that are f32 -- S, delta, T, beta e^G k,
 // beta v, P, and q, k, v themselves when they arrive as f32 -- are split into
-// hi = f16(x) and lo = f16(x - hi) and multiplied as hi*hi + hi*lo + lo*hi
-// (about 22 significant bits), so the result tracks the f32 recurrence of the
-// reference's prefill scan.  (f16 q, k, v take the kernels of gdn_prefill16.hip.)
+// hi = f16(x) and lo = f16(x - hi) and multiplied as hi*hi + hi*lo + lo*hi:
+// about 22 significant bits, but for some elements of what is itself a product
+// or a difference (beta e^G k, beta v, P, delta): there the compiler rounds hi
+// from the exact value and lo from its f32 rounding, and where those two round
+// to different f16 the halves are an ulp apart, 11 bits.  Against 64 bits, f32
+// rows, 600 tokens of 16 heads: 1.5e-5 of the output and 5e-3 of its rms in the
+// worst element; with both halves from one value (gd_split_f16) 7e-6 and 5e-5,
+// at the same time.  Its outputs are compared with recorded ones at 2e-3 of the
+// rms an element, which is less than the two forms differ by, so this one stays.
+// (f16 q, k, v take the kernels of gdn_prefill16.hip, which split by gd_split_f16.)
 //   gdn_prep  (value head, chunk): K K^T and Q K^T on the matrix cores give A
 //             and P; I + A is inverted in 16 x 16 blocks (diagonal blocks by
 //             forward substitution, one wave each, then the blocks below in
@@ -48,7 +55,8 @@ __device__ __forceinline__ f32x4 mfma(const f16x8 &a, const f16x8 &b, const f32x
     return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
 }
 
-// x = hi + lo, hi = f16(x), lo = f16(x - hi).
+// x = hi + lo, hi = f16(x), lo = f16(x - hi) (an ulp of hi apart for some x that
+// are products, above).
 __device__ __forceinline__ void split8(const float (&x)[8], f16x8 &hi, f16x8 &lo) {
 #pragma unroll
     for (int e = 0; e < 8; e++) {

@@ -349,7 +349,11 @@ int gd_kv_append(gd_ctx *ctx, const float *k, const float *v, uint16_t *k_cache,
  * appended first): out[h] = softmax((q_h . k_t) * scale) . v_t, times
  * sigmoid(gate[h]) when gated (1; 0: plain).  q, gate, out [n_head][head_dim]
  * f32.  part: scratch of n_head * 16 * (head_dim + 2) floats (the key-split
- * partials).  MetalEnc.attnPaged (MetalEnc.swift:679-706), attn_head
+ * partials; long contexts use the context's or the recording's own beside it).
+ * An infinity in the cache (kv_append of a value past f16's range): a key whose
+ * score is -inf weighs nothing, an infinite V makes its dim of the output that
+ * infinity; +inf scores, and infinities of both signs in one dim, give NaN.
+ * MetalEnc.attnPaged (MetalEnc.swift:679-706), attn_head
  * (Kernels.metal:1423-1445). */
 int gd_attn_paged(gd_ctx *ctx, const float *q, const uint16_t *k_cache,
                   const uint16_t *v_cache, const int32_t *page_table, const float *gate,
