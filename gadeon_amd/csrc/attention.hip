@@ -27,8 +27,8 @@
 //     K and V as stored, V^T taken by the transposing LDS read; S^T = K Q^T
 //     and O^T += V^T P^T on v_mfma_f32_16x16x32_f16 with the key order
 //     inside the MFMA K dimension permuted so that P stays in registers; q
-//     and P as f16 hi + lo pairs (about 22 bits), K and V the f16 cache, f32
-//     accumulation.  In the stack the prefill normalizes and rotates q from
+//     and P as f16 hi + lo pairs (about 22 bits, but for some q of head dim
+//     128, at its split), K and V the f16 cache, f32 accumulation.  In the stack the prefill normalizes and rotates q from
 //     the projection rows itself and prep handles the kv heads only.
 #include "gd_internal.h"
 

@@ -148,7 +148,7 @@ def test_decode_and_batch_attention(ctx, hd, nh, nkv, page, T):
 def test_decode_attention_key_blocks(ctx, hd, nh, nkv, page, T, lo):
     """One query over cached keys lo .. T-1 around the edges of the key blocks
     and splits (one key, one past a block, several rounds of a wave) and of the
-    few keys (9/2 head dims) that go a wave a key, with one, two, five, six
+    few keys that go a wave a key, with one, two, five, six
     and more than eight q heads a kv head: against f64 over the same f16 cache
     within 3e-6 (22-bit q and weights, f32 sums)."""
     rng = np.random.default_rng(T + nh)
