@@ -268,8 +268,9 @@ __global__ __launch_bounds__(256) void k_attn_prefill(
     // 3584 keys, 40 / 8 heads, against 64 bits: 3.2e-6 of the output, 6e-4 of its
     // rms in the worst element; by gd_split_f16 7e-7 and 2e-5, at the same time.
     // Its outputs are compared with recorded ones at 4e-4 of the rms an element,
-    // less than the two forms differ by, so it stays; head dim 256's scale 1/16 is
-    // exact either way, and its other scales keep 22 bits.
+    // less than the two forms differ by, so it stays.  Head dim 256 splits by
+    // gd_split_f16, but for scales that are powers of two, as 1/16: those products
+    // are exact either way, and the fence costs 0.5 us of a short call's 23.
     const int64_t qoff = (int64_t)(valid ? n : N - 1) * qsrc.tstride + (int64_t)h * qsrc.hstride;
     f16x8 qh[HD / 32], ql[HD / 32];
     {
@@ -315,26 +316,26 @@ __global__ __launch_bounds__(256) void k_attn_prefill(
                 }
             }
         }
+        if (HD == 256 && (__float_as_uint(scale) & 0x7fffffu)) {
 #pragma unroll
-        for (int ks = 0; ks < HD / 32; ks++)
+            for (int ks = 0; ks < HD / 32; ks++)
 #pragma unroll
-            for (int e = 0; e < 8; e += 2) {
-                const float v[2] = {x[ks][e] * scale, x[ks][e + 1] * scale};
-                if constexpr (HD == 256) {
-                    f16x2 hi, lo;
-                    gd_split2_f16(v[0], v[1], hi, lo);
-                    qh[ks][e] = hi[0];
-                    qh[ks][e + 1] = hi[1];
-                    ql[ks][e] = lo[0];
-                    ql[ks][e + 1] = lo[1];
-                } else {
-#pragma unroll
-                    for (int i = 0; i < 2; i++) {
-                        qh[ks][e + i] = (f16)v[i];
-                        ql[ks][e + i] = (f16)(v[i] - (float)qh[ks][e + i]);
-                    }
+                for (int e = 0; e < 8; e++) {
+                    f16 hi, lo;
+                    gd_split_f16(x[ks][e] * scale, hi, lo);
+                    qh[ks][e] = hi;
+                    ql[ks][e] = lo;
                 }
-            }
+        } else {
+#pragma unroll
+            for (int ks = 0; ks < HD / 32; ks++)
+#pragma unroll
+                for (int e = 0; e < 8; e++) {
+                    const float v = x[ks][e] * scale;
+                    qh[ks][e] = (f16)v;
+                    ql[ks][e] = (f16)(v - (float)qh[ks][e]);
+                }
+        }
     }
     f32x4 acc[HD / 16];                                   // O^T rows 16 dt + 4 g + v
 #pragma unroll
