@@ -35,6 +35,15 @@ def chain_ms(ctx, call, n=50, replays=12):
     return best
 
 
+def not_slower(ctx, picked, other, n=50):
+    """Chains of the two calls, measured again where something else ran beside one."""
+    for _ in range(3):
+        a, b = chain_ms(ctx, picked, n), chain_ms(ctx, other, n)
+        if a < SLACK * b:
+            return
+    assert a < SLACK * b
+
+
 def zeros(ctx, nbytes):
     p = ctx.alloc(nbytes)
     ctx.gd_fill_u32(p, 0, nbytes // 4)
@@ -47,9 +56,8 @@ def test_conv_few_tokens(ctx, N):
     output replaces its input."""
     cd = 8192
     x, o, ring, cw = (zeros(ctx, n * cd * 4) for n in (N, N, 3, 4))
-    picked = chain_ms(ctx, lambda: ctx.gd_gdn_conv(x, ring, cw, o, cd, 4, N))
-    serial = chain_ms(ctx, lambda: ctx.gd_gdn_conv(x, ring, cw, x, cd, 4, N))
-    assert picked < SLACK * serial
+    conv = lambda out: ctx.gd_gdn_conv(x, ring, cw, out, cd, 4, N)
+    not_slower(ctx, lambda: conv(o), lambda: conv(x))
     for p in (x, o, ring, cw):
         ctx.free(p)
 
@@ -58,9 +66,8 @@ def test_conv_few_tokens(ctx, N):
 def test_rmsnorm_rows_few(ctx, d, rows):
     """Few rows, and many, against the kernel for any alignment (w one float off)."""
     x, w = zeros(ctx, rows * d * 4), zeros(ctx, d * 4 + 16)
-    picked = chain_ms(ctx, lambda: ctx.gd_rmsnorm_rows(x, d, rows, w, EPS))
-    general = chain_ms(ctx, lambda: ctx.gd_rmsnorm_rows(x, d, rows, w + 4, EPS))
-    assert picked < SLACK * general
+    norm = lambda weights: ctx.gd_rmsnorm_rows(x, d, rows, weights, EPS)
+    not_slower(ctx, lambda: norm(w), lambda: norm(w + 4))
     for p in (x, w):
         ctx.free(p)
 
@@ -69,9 +76,8 @@ def test_rmsnorm_rows_few(ctx, d, rows):
 def test_rmsnorm_short_rows(ctx, n, rows):
     """Many short rows against the kernel for any alignment (w one float off)."""
     x, w, y = zeros(ctx, rows * n * 4), zeros(ctx, n * 4 + 16), zeros(ctx, rows * n * 4)
-    picked = chain_ms(ctx, lambda: ctx.gd_rmsnorm(x, w, y, ga.F32, n, rows, EPS), 20)
-    general = chain_ms(ctx, lambda: ctx.gd_rmsnorm(x, w + 4, y, ga.F32, n, rows, EPS), 20)
-    assert picked < SLACK * general
+    norm = lambda weights: ctx.gd_rmsnorm(x, weights, y, ga.F32, n, rows, EPS)
+    not_slower(ctx, lambda: norm(w), lambda: norm(w + 4), 20)
     for p in (x, w, y):
         ctx.free(p)
 
@@ -100,8 +106,7 @@ def test_decode_attention_keys(ctx, hd, nh, nkv, T):
     q, gate, out, part = (zeros(ctx, n * 4 + 16) for n in (nh * hd, nh * hd, nh * hd, nh * 16 * (hd + 2)))
     call = lambda x: ctx.gd_attn_paged(x, kc, vc, table, gate, out, part, hd, nh, nkv, T, kv_dim, page,
                                        C.c_float(hd ** -0.5), 1, 0)
-    picked = chain_ms(ctx, lambda: call(q))
-    assert picked < SLACK * chain_ms(ctx, lambda: call(q + 4))
+    not_slower(ctx, lambda: call(q), lambda: call(q + 4))
     for p in (kc, vc, table, q, gate, out, part):
         ctx.free(p)
 
@@ -118,9 +123,8 @@ def weights(ctx, K, R):
 def test_swiglu_few_tokens(ctx, T, K, ff):
     """Few tokens at every K and ff against the tiles, which a forced plan takes."""
     w, x, o = weights(ctx, K, 2 * ff), zeros(ctx, T * K * 2), zeros(ctx, T * ff * 2)
-    picked = chain_ms(ctx, lambda: ctx.gd_q2_0_gemm_swiglu(C.byref(w), T, x, o), 20)
-    tiles = chain_ms(ctx, lambda: ctx.gd_q2_0_gemm_swiglu_plan(C.byref(w), T, x, o, 0), 20)
-    assert picked < SLACK * tiles
+    not_slower(ctx, lambda: ctx.gd_q2_0_gemm_swiglu(C.byref(w), T, x, o),
+               lambda: ctx.gd_q2_0_gemm_swiglu_plan(C.byref(w), T, x, o, 0), 20)
     ctx.gd_q2w_free(C.byref(w))
     for p in (x, o):
         ctx.free(p)
@@ -130,9 +134,8 @@ def test_swiglu_few_tokens(ctx, T, K, ff):
 def test_gemm_few_tokens_plan(ctx, T, K, R):
     """Few tokens at every K against a tile that needs no K split."""
     w, x, o = weights(ctx, K, R), zeros(ctx, T * K * 2), zeros(ctx, T * R * 4)
-    picked = chain_ms(ctx, lambda: ctx.gd_q2_0_gemm(C.byref(w), T, x, ga.F16, o, ga.F32), 20)
-    tiles = chain_ms(ctx, lambda: ctx.gd_q2_0_gemm_plan(C.byref(w), T, x, ga.F16, o, ga.F32, 1, 1, 1, 4), 20)
-    assert picked < SLACK * tiles
+    not_slower(ctx, lambda: ctx.gd_q2_0_gemm(C.byref(w), T, x, ga.F16, o, ga.F32),
+               lambda: ctx.gd_q2_0_gemm_plan(C.byref(w), T, x, ga.F16, o, ga.F32, 1, 1, 1, 4), 20)
     ctx.gd_q2w_free(C.byref(w))
     for p in (x, o):
         ctx.free(p)
