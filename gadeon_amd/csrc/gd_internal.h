@@ -41,7 +41,7 @@ struct gd_ctx {
     // Inside a recording (gd_graph_begin .. gd_graph_end): what the graph will
     // hold, the workspace if an entry used it and attention partials of its own,
     // since it may be launched beside this context's calls and outlive them.
-    bool recording = false;
+    bool recording = false, rec_failed = false;
     gd_buf *rec_ws = nullptr, *rec_attn = nullptr;
     std::string err;
 };

@@ -121,8 +121,13 @@ void gd_buf_drop(gd_buf *b) {
 
 int gd_ctx_workspace(gd_ctx *ctx, size_t bytes, void **out) {
     if (ctx->ws_bytes < bytes) {
-        // Inside a recording this fails, and the recording with it.
-        if (ctx->ws || ctx->recording) GD_HIP(ctx, hipStreamSynchronize(ctx->stream));
+        // Inside a recording this fails, and the recording with it (a HIP call
+        // that fails in a capture would leave the stream unusable).
+        if (ctx->recording) {
+            ctx->rec_failed = true;
+            return gd_fail(ctx, GD_ENOMEM, "workspace (%zu bytes) would grow inside a recording", bytes);
+        }
+        if (ctx->ws) GD_HIP(ctx, hipStreamSynchronize(ctx->stream));
         gd_buf_drop(ctx->ws);
         ctx->ws_bytes = 0;
         ctx->ws = gd_buf_new(bytes);
@@ -267,6 +272,7 @@ extern "C" int gd_graph_begin(gd_ctx *ctx) {
     GD_CHECK_CTX(ctx);
     GD_HIP(ctx, hipStreamBeginCapture(ctx->stream, hipStreamCaptureModeThreadLocal));
     ctx->recording = true;
+    ctx->rec_failed = false;
     return GD_OK;
 }
 
@@ -281,6 +287,10 @@ extern "C" int gd_graph_end(gd_ctx *ctx, gd_graph **out) {
     if (e != hipSuccess) {
         gd_graph_destroy(g);
         return gd_hip_fail(ctx, e, "gd_graph_end: hipStreamEndCapture");
+    }
+    if (ctx->rec_failed) {
+        gd_graph_destroy(g);
+        return gd_fail(ctx, GD_EHIP, "gd_graph_end: a call inside the recording failed for lack of workspace (capture discarded)");
     }
     if (!out) {
         gd_graph_destroy(g);

@@ -718,6 +718,34 @@ def test_gemv_norm_large_norm_weight(ctx):
     free_w(ctx, w)
 
 
+@pytest.mark.parametrize("warm", [False, True])
+def test_graph_refuses_workspace_growth(warm):
+    """An entry that needs a (larger) workspace inside a recording fails, and so
+    does the recording's end; the context then works and records again."""
+    K, R = 512, 96
+    with ga.Context(0) as c:
+        w = upload_w(c, O.lcg_q2_0(K, R, 4), K, R)
+        X = O.lcg_normal(64 * K, 5).astype(np.float32).reshape(64, K)
+        dX, dY, g = c.put(X), c.alloc(64 * R * 4), C.c_void_p()
+        call = lambda T: c.gd_q2_0_gemm(C.byref(w), T, dX, ga.F32, dY, ga.F32)
+        if warm:
+            call(4)
+        c.gd_graph_begin()
+        with pytest.raises(ga.GDError):
+            call(64)
+        assert c.lib.gd_graph_end(c.h, C.byref(g)) != 0 and not g.value
+        call(64)
+        want = c.get(dY, 64 * R, np.float32)
+        c.gd_fill_u32(dY, 0, 64 * R)
+        c.gd_graph_begin()
+        call(64)
+        c.gd_graph_end(C.byref(g))
+        c.gd_graph_launch(g)
+        assert np.array_equal(c.get(dY, 64 * R, np.float32), want)
+        c.lib.gd_graph_destroy(g)
+        free_w(c, w)
+
+
 def test_graph_replays_recorded_calls(ctx):
     """gd_graph_begin/end record GEMVs on three distinct matrices and a cast;
     each replay, with eager work and synchronizations in between, gives the
